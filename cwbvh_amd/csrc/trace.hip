@@ -147,7 +147,8 @@ struct CwbvhParams {
     unsigned long long* stats;      // {nodes, triangles}
     int n;                          // rays (single) or total chunks (multi)
     int slices;                     // single scene: contiguous ray ranges, one per XCD
-    int persistent;                 // 0: one ray per thread, no refill
+    int persistent;                 // 0: each wave traces rays_per_wave rays, no refill
+    int rays_per_wave;              // persistent 0: rays given to a wave, 1..64
     int num_jobs;
     int stride;                     // float4 per node: 5 or 8
     int lds_depth;
@@ -247,15 +248,257 @@ constexpr int kLoopQueue = 3;
 // instances stay unconstrained: the batch, counting and prefetching kernels
 // spill 10 to 32 registers at 7 waves, and the grouped and speculative
 // schedules serve scenes that stream from HBM, where spills and the extra
-// wave cost more.
+// wave cost more.  The LDS-only build that reads rays from a buffer is held to
+// 6 waves: team_trace's code would lift it from 76 to 83 VGPRs, i.e. to 5; held,
+// it takes 77-79 and spills nothing.
 constexpr int kOccupancyAuto = 0;
 constexpr int kOccupancyFree = 1;
 constexpr int kOccupancy7 = 7;
 constexpr long long kOccupancy7MinRays = 1ll << 22;  // automatic choice: launches this large
 
 #ifndef CWBVH_TRACE_ATTR
-#define CWBVH_TRACE_ATTR __attribute__((amdgpu_waves_per_eu(W7 ? 7 : 1)))
+#define CWBVH_TRACE_ATTR __attribute__((amdgpu_waves_per_eu(W7 ? 7 : (LDSO && !MULTI && !PREFETCH && SRC == 0) ? 6 : 1)))
 #endif
+
+// A wave whose pool is dry traces its last kLastRays rays with teams of lanes
+// (team_trace): 4 lanes per ray, and 8 once 8 rays are left.
+constexpr int kLastRays = 16;
+
+// A value of the other lane of each pair, the other pair of each quad, and the
+// other quad of each 8 lanes (DPP quad_perm [1,0,3,2], quad_perm [2,3,0,1],
+// row_half_mirror): two (teams of 4) or three (teams of 8) steps of an
+// associative, commutative operation leave its result over the team in all of
+// its lanes.
+constexpr int kDppPair = 0xB1, kDppQuad = 0x4E, kDppHalf = 0x141;
+template <int CTRL>
+__device__ __forceinline__ int team_swap(int v) {
+    return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, false);
+}
+
+template <int TEAM>
+__device__ __forceinline__ unsigned team_or(unsigned v) {
+    v |= (unsigned)team_swap<kDppPair>((int)v);
+    v |= (unsigned)team_swap<kDppQuad>((int)v);
+    if (TEAM == 8) v |= (unsigned)team_swap<kDppHalf>((int)v);
+    return v;
+}
+
+// The lower (t, address) of two candidates.
+template <int CTRL>
+__device__ __forceinline__ void team_min_step(float& t, int& a) {
+    const float ot = i2f(team_swap<CTRL>(f2i(t)));
+    const int oa = team_swap<CTRL>(a);
+    const bool take = ot < t || (ot == t && oa < a);
+    t = take ? ot : t;
+    a = take ? oa : a;
+}
+
+// One ray's traversal state, as cwbvh_trace holds it per lane.
+struct RayState {
+    float3 o, d;
+    float tmin, tmax, idx, idy, idz;
+    unsigned octinv;
+    uint2 ng, tg;
+    int sp, col, hit_addr, out_idx;   // col: the ray's stack column in LDS
+    unsigned out_texel;
+    float hu, hv;
+    const float4* nodes;
+    const float4* tris;
+    float4* hits;
+    const int* prim_map;
+    unsigned stride_sh;
+};
+
+template <class T>
+__device__ __forceinline__ T* shfl_ptr(T* p, int src) {
+    return (T*)__shfl((unsigned long long)p, src);
+}
+
+template <int SRC, bool MULTI>
+__device__ __forceinline__ void shfl_state(RayState& r, int src) {
+    r.o.x = __shfl(r.o.x, src); r.o.y = __shfl(r.o.y, src); r.o.z = __shfl(r.o.z, src);
+    r.d.x = __shfl(r.d.x, src); r.d.y = __shfl(r.d.y, src); r.d.z = __shfl(r.d.z, src);
+    r.tmin = __shfl(r.tmin, src); r.tmax = __shfl(r.tmax, src);
+    r.idx = __shfl(r.idx, src); r.idy = __shfl(r.idy, src); r.idz = __shfl(r.idz, src);
+    r.octinv = __shfl(r.octinv, src);
+    r.ng.x = __shfl(r.ng.x, src); r.ng.y = __shfl(r.ng.y, src);
+    r.tg.x = __shfl(r.tg.x, src); r.tg.y = __shfl(r.tg.y, src);
+    r.sp = __shfl(r.sp, src); r.col = __shfl(r.col, src);
+    r.hit_addr = __shfl(r.hit_addr, src); r.out_idx = __shfl(r.out_idx, src);
+    r.hu = __shfl(r.hu, src); r.hv = __shfl(r.hv, src);
+    if constexpr (SRC == kRaysFromSurfels) r.out_texel = __shfl(r.out_texel, src);
+    if constexpr (MULTI) {
+        r.nodes = shfl_ptr(r.nodes, src);
+        r.tris = shfl_ptr(r.tris, src);
+        r.hits = shfl_ptr(r.hits, src);
+        r.prim_map = shfl_ptr(r.prim_map, src);
+        r.stride_sh = __shfl(r.stride_sh, src);
+    }
+}
+
+// Writes a finished ray's hit, or counts it on its surfel.
+template <int SRC>
+__device__ __forceinline__ void write_hit(const CwbvhParams& P, const RayState& r) {
+    if (SRC == kRaysFromSurfels && P.texel_hits) {
+        if (r.hit_addr >= 0) atomicAdd(&P.texel_hits[r.out_texel], 1u);
+    } else {
+        const int out_id = (r.hit_addr >= 0 && P.prim_id) ? r.prim_map[r.hit_addr] : r.hit_addr;
+        nt_store4(make_float4(r.tmax, i2f(out_id), r.hu, r.hv), &r.hits[r.out_idx]);
+    }
+}
+
+// Traces a wave's remaining rays (lanes `live`, at most 64 / TEAM of them)
+// with a team of TEAM lanes per ray until at most `leave` are left; returns
+// the lanes that hold those (the first lane of each team).  All 64 lanes call
+// it, each with its own ray state in `r`.
+//
+// The last rays of a wave are chains of dependent node loads and of the ~320
+// instructions between them, issued for a few lanes: about 1 us per visit, so a
+// launch lasts as long as its slowest rays however few they are.  Here lane j of
+// a team tests 8 / TEAM children of the node and one triangle of the group,
+// which cuts the chain per visit to the load and about 90 instructions.
+// The visits, the tests and their arithmetic are those of the one-lane
+// schedule, so the hits are too: a triangle group's closest hit is its lowest
+// (t, address) under the same tie rule, its any hit the accepted triangle with
+// the highest bit.  The stack stays in the LDS column of the ray's first lane.
+template <bool ANY, int SRC, bool MULTI, int TEAM>
+__device__ __forceinline__ unsigned long long team_trace(const CwbvhParams& P, CWD_LDS unsigned long long* lds_stack,
+                                                         unsigned long long live, int leave, int lane, RayState& r) {
+    constexpr int kChildren = 8 / TEAM;   // children per lane: j and, teams of 4, j + 4
+    const int team = (int)((unsigned)lane / TEAM), j = (int)((unsigned)lane % TEAM);
+    int src = 0;
+    const int count = __popcll(live);
+    for (int k = 0; k < count; ++k) {
+        const int s = __ffsll((long long)live) - 1;
+        live &= live - 1ull;
+        if (team == k) src = s;
+    }
+    shfl_state<SRC, MULTI>(r, src);
+    bool busy = team < count;
+    if (busy) {
+        const int tx = r.idx < 0.f ? 24 : 0, ty = r.idy < 0.f ? 24 : 0, tz = r.idz < 0.f ? 24 : 0;
+        while (true) {
+            if (r.tg.y == 0u && r.ng.y > 0x00FFFFFFu) {
+                const unsigned imask = r.ng.y;
+                const int bit = 31 - __clz((int)r.ng.y);
+                const unsigned slot = (unsigned)(bit - 24) ^ r.octinv;
+                const unsigned rel = (unsigned)__popc(imask & ~(0xFFFFFFFFu << slot));
+                const float4* np = node_at(r.nodes, r.ng.x + rel, r.stride_sh);
+                // this lane's planes: bytes lo x, y, z, hi x, y, z of 8 children each
+                const unsigned char* q = reinterpret_cast<const unsigned char*>(np + 2) + j;
+                const float4 n0 = np[0], n1 = np[1];
+                unsigned near[kChildren][3], far[kChildren][3];
+#pragma unroll
+                for (int c = 0; c < kChildren; ++c) {
+                    near[c][0] = q[tx + 4 * c];
+                    near[c][1] = q[8 + ty + 4 * c];
+                    near[c][2] = q[16 + tz + 4 * c];
+                    far[c][0] = q[24 - tx + 4 * c];
+                    far[c][1] = q[32 - ty + 4 * c];
+                    far[c][2] = q[40 - tz + 4 * c];
+                }
+                r.ng.y &= ~(1u << bit);
+                if (r.ng.y > 0x00FFFFFFu) {
+                    if (r.sp < P.lds_depth) {
+                        lds_stack[(r.sp << 6) + r.col] = pack2(r.ng);
+                        ++r.sp;
+                    } else {
+                        P.work[kWorkOverflow] = 1u;
+                    }
+                }
+                const unsigned eb = f2u(n0.w);
+                const int ex = (int)(signed char)(eb & 0xFFu);
+                const int ey = (int)(signed char)((eb >> 8) & 0xFFu);
+                const int ez = (int)(signed char)((eb >> 16) & 0xFFu);
+                const float adjx = u2f((unsigned)(ex + 127) << 23) * r.idx;
+                const float adjy = u2f((unsigned)(ey + 127) << 23) * r.idy;
+                const float adjz = u2f((unsigned)(ez + 127) << 23) * r.idz;
+                const float origx = -(r.o.x - n0.x) * r.idx;
+                const float origy = -(r.o.y - n0.y) * r.idy;
+                const float origz = -(r.o.z - n0.z) * r.idz;
+                unsigned hitmask = 0;
+#pragma unroll
+                for (int c = 0; c < kChildren; ++c) {
+                    const float tnx = __builtin_fmaf((float)near[c][0], adjx, origx);
+                    const float tny = __builtin_fmaf((float)near[c][1], adjy, origy);
+                    const float tnz = __builtin_fmaf((float)near[c][2], adjz, origz);
+                    const float tfx = __builtin_fmaf((float)far[c][0], adjx, origx);
+                    const float tfy = __builtin_fmaf((float)far[c][1], adjy, origy);
+                    const float tfz = __builtin_fmaf((float)far[c][2], adjz, origz);
+                    const float cmin = imax2(imax3(tnx, tny, tnz), r.tmin);
+                    const float cmax = imin2(imin3(tfx, tfy, tfz), r.tmax);
+                    const unsigned meta4 = (TEAM == 8 ? j < 4 : c == 0) ? f2u(n1.z) : f2u(n1.w);
+                    const unsigned meta = (meta4 >> (8 * (j & 3))) & 0xFFu;
+                    const bool inner = (meta & (meta << 1) & 0x10u) != 0u;
+                    const unsigned at = (meta ^ (inner ? r.octinv : 0u)) & 0x1Fu;
+                    hitmask |= cmin <= cmax ? (meta >> 5) << at : 0u;
+                }
+                hitmask = team_or<TEAM>(hitmask);
+                r.ng = make_uint2(f2u(n1.x), (hitmask & 0xFF000000u) | (eb >> 24));
+                r.tg = make_uint2(f2u(n1.y), hitmask & 0x00FFFFFFu);
+            }
+            bool finished = false;
+            while (r.tg.y != 0u) {
+                // lane j takes the (j + 1)-th highest triangle of the group
+                int mine = -1;
+                for (int k = 0; k < TEAM && r.tg.y != 0u; ++k) {
+                    const int h = 31 - __clz((int)r.tg.y);
+                    mine = j == k ? h : mine;
+                    r.tg.y &= ~(1u << h);
+                }
+                bool ok = false;
+                int addr = 0;
+                float t = 0.f, u = 0.f, v = 0.f;
+                if (mine >= 0) {
+                    addr = (int)(r.tg.x * 3u + (unsigned)mine * 3u);
+                    const float4 v0 = r.tris[addr], v1 = r.tris[addr + 1], v2 = r.tris[addr + 2];
+                    ok = woop_test<ANY>(v0, v1, v2, r.o, r.d, r.tmin, r.tmax, addr, r.hit_addr, t, u, v);
+                }
+                if constexpr (ANY) {
+                    // the first accepted triangle in the group's order
+                    const unsigned m = (unsigned)(__ballot(ok) >> (team * TEAM)) & ((1u << TEAM) - 1u);
+                    if (m != 0u) {
+                        const int w = team * TEAM + __ffs((int)m) - 1;
+                        r.tmax = __shfl(t, w);
+                        r.hit_addr = __shfl(addr, w);
+                        r.hu = __shfl(u, w);
+                        r.hv = __shfl(v, w);
+                        finished = true;
+                        break;
+                    }
+                } else {
+                    float bt = ok ? t : INFINITY;
+                    int ba = ok ? addr : 0x7FFFFFFF;
+                    team_min_step<kDppPair>(bt, ba);
+                    team_min_step<kDppQuad>(bt, ba);
+                    if (TEAM == 8) team_min_step<kDppHalf>(bt, ba);
+                    if (ba != 0x7FFFFFFF) {
+                        const bool won = ok && addr == ba;
+                        r.tmax = bt;
+                        r.hit_addr = ba;
+                        r.hu = u2f(team_or<TEAM>(won ? f2u(u) : 0u));
+                        r.hv = u2f(team_or<TEAM>(won ? f2u(v) : 0u));
+                    }
+                }
+            }
+            if (!finished && r.ng.y <= 0x00FFFFFFu) {
+                if (r.sp > 0) {
+                    --r.sp;
+                    r.ng = unpack2(lds_stack[(r.sp << 6) + r.col]);
+                } else {
+                    finished = true;
+                }
+            }
+            if (finished) {
+                if (j == 0) write_hit<SRC>(P, r);
+                busy = false;
+                break;
+            }
+            if (__popcll(__ballot(j == 0)) <= leave) break;
+        }
+    }
+    return __ballot(busy && j == 0);
+}
 
 template <bool ANY, bool STATS, bool MULTI, bool PREFETCH, int LOOP, int SRC = kRaysFromBuffer, bool W7 = false,
           bool LDSO = false>
@@ -266,6 +509,11 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
     // lds_depth stack entries, so the stack lives in LDS only (interleaved
     // schedule: only node groups are pushed, one per level of the tree)
     static_assert(!LDSO || (LOOP == kLoopInterleave && !STATS), "LDS-only stacks serve the interleaved schedule");
+    // The last rays of a wave go to teams of lanes (team_trace) where the stack
+    // is in LDS.  The 7-wave builds serve launches of 2^22 rays and more, whose
+    // tail is 3% of their time; with team_trace their node loop spills scalars
+    // and they run 2.3% slower (33 M AO rays: 2.19 against 2.14 ms).
+    constexpr bool kTeams = LDSO && !W7;
     extern __shared__ unsigned long long lds_stack_raw[];
     CWD_LDS unsigned long long* lds_stack = lds_ptr(lds_stack_raw);
     unsigned long long spill[kStackCapacity];
@@ -332,19 +580,13 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                 if (exhausted) break;
                 const int leader = __ffsll((long long)need) - 1;
                 if (!MULTI && !P.persistent) {
-                    // one ray per thread: the only "pool" is this wave's own 64 indices
-                    if (slice_k > 0) {
-                        exhausted = true;
-                        break;
-                    }
-                    slice_k = 1;
-                    const unsigned first = (blockIdx.x * blockDim.x + (threadIdx.x & ~63u));
+                    // no work fetching: the only "pool" is this wave's own rays_per_wave indices
+                    exhausted = true;
+                    const unsigned share = kTeams ? (unsigned)P.rays_per_wave : 64u;
+                    const unsigned first = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * share;
                     pool_next = min(first, (unsigned)P.n);
-                    pool_end = min(first + 64u, (unsigned)P.n);
-                    if (pool_next >= pool_end) {
-                        exhausted = true;
-                        break;
-                    }
+                    pool_end = min(first + share, (unsigned)P.n);
+                    if (pool_next >= pool_end) break;
                 } else if (MULTI) {
                     // claim one chunk index from the home slice of the chunk
                     // range, then from the others
@@ -419,7 +661,6 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
             pool_next += min((unsigned)__popcll(need), avail);
             need = __ballot(terminated && !got);
         }
-        if (terminated && !got) break;  // no work left for this lane
 
         if (got) {
             const Ray4* rays = P.rays;
@@ -475,6 +716,13 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
             hu = hv = 0.f;
             have_pf = false;
             busy = true;
+        }
+
+        if constexpr (kTeams) {
+            if (exhausted && __popcll(__ballot(busy)) <= kLastRays) break;
+            if (!busy) continue;  // idle until the wave ends
+        } else {
+            if (terminated && !got) break;  // no work left for this lane
         }
 
         // stack push of a node or triangle group (overflow is flagged, not written)
@@ -678,11 +926,26 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                 busy = false;
                 break;
             }
-            lost += __popcll(~__ballot(1)) - P.idle_lanes;
-            if (lost >= P.idle_budget) break;
+            const int idle = __popcll(~__ballot(1));
+            lost += idle - P.idle_lanes;
+            if constexpr (kTeams) {
+                if (exhausted ? idle >= 64 - kLastRays : lost >= P.idle_budget) break;
+            } else {
+                if (lost >= P.idle_budget) break;
+            }
         }
     }
 
+    if constexpr (kTeams) {
+        // the last rays of the wave, with teams of lanes
+        unsigned long long live = __ballot(busy);
+        if (live != 0ull) {
+            RayState r{o, d, tmin, tmax, idx, idy, idz, octinv, ng, tg, sp, sx.col, hit_addr, out_idx,
+                       out_texel, hu, hv, nodes, tris, hits, prim_map, stride_sh};
+            if (__popcll(live) > 8) live = team_trace<ANY, SRC, MULTI, 4>(P, lds_stack, live, 8, lane, r);
+            team_trace<ANY, SRC, MULTI, 8>(P, lds_stack, live, 0, lane, r);
+        }
+    }
     if (STATS) {
         atomicAdd(&P.stats[0], st_nodes);
         atomicAdd(&P.stats[1], st_tris);
@@ -1153,7 +1416,22 @@ int32_t launch_cwbvh_t(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStream_
     auto kernel = cwbvh_trace<ANY, STATS, MULTI, PREFETCH, LOOP, SRC, W7, LDSO>;
     long long grid = cfg.grid_blocks;
     if (!MULTI && !p.persistent) {
-        grid = ((long long)p.n + block - 1) / block;
+        // Waves of the LDS-only kernels trace their last 16 rays with 4 or 8
+        // lanes each (team_trace), so a launch too small to fill the device
+        // gives each wave only 8 or 16 rays: one latency chain per ray shrinks
+        // from the start.  The limit is 4 waves per SIMD; with more, the teams'
+        // waves queue behind one another (MI355X, AO rays on a 65 k-triangle
+        // heightfield, closest hit, us for 64 / 16 / 8 rays per wave: 1,000
+        // rays 37 / 32 / 21; 32,000 rays 36 / 32 / 28; 48,000 rays 35 / 32 / 43;
+        // 96,000 rays 40 / 69 / 63)
+        p.rays_per_wave = 64;
+        if (LDSO && !W7) {
+            const long long waves = 16ll * cw::device_compute_units();
+            if ((p.n + 7) / 8 <= waves) p.rays_per_wave = 8;
+            else if ((p.n + 15) / 16 <= waves) p.rays_per_wave = 16;
+        }
+        const long long per_block = (long long)p.rays_per_wave * (block / 64);
+        grid = ((long long)p.n + per_block - 1) / per_block;
         p.idle_budget = 0x7FFFFFFF;  // nothing to refill from
     } else if (grid <= 0) {
         grid = (long long)resident_blocks(kernel, block, lds) * cw::device_compute_units();
