@@ -326,12 +326,25 @@ int32_t cwbvh_scene_create_ex(const cwbvh_layout* L, void* stream, int32_t strid
     // read of the last leaf inside the allocation
     const size_t wb = (L->woop.size() + 2) * sizeof(cwbvh_float4);
     const size_t pb = std::max<size_t>(1, L->prim_idx.size()) * sizeof(int32_t);
-    void *dn = nullptr, *dw = nullptr, *dp = nullptr;
+    const int64_t num_nodes = L->kind == CWBVH_KIND_CWBVH ? (int64_t)(node_f4 / (size_t)stride) : 0;
+    void *dn = nullptr, *dw = nullptr, *dp = nullptr, *ds = nullptr;
     hipError_t e = hipMalloc(&dn, nb);
     if (e == hipSuccess) e = hipMalloc(&dw, wb);
     if (e == hipSuccess) e = hipMalloc(&dp, pb);
+    // 128 B nodes: also the spread copy that the LDS-only kernels read (without
+    // room for it they read the nodes themselves)
+    size_t sb = 0;
+    if (e == hipSuccess && L->kind == CWBVH_KIND_CWBVH && stride == 8 && num_nodes <= kMaxSpreadNodes) {
+        sb = (size_t)num_nodes * 128;
+        if (hipMalloc(&ds, sb) != hipSuccess) {
+            (void)hipGetLastError();
+            ds = nullptr;
+            sb = 0;
+        }
+    }
     hipStream_t st = (hipStream_t)stream;
     if (e == hipSuccess) e = hipMemcpyAsync(dn, node_src, nb, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess && ds && launch_spread_nodes(dn, num_nodes, stride, ds, st) != CWBVH_OK) e = hipErrorLaunchFailure;
     if (e == hipSuccess) e = hipMemsetAsync(dw, 0, wb, st);
     if (e == hipSuccess && !L->woop.empty())
         e = hipMemcpyAsync(dw, L->woop.data(), L->woop.size() * sizeof(cwbvh_float4), hipMemcpyHostToDevice, st);
@@ -342,12 +355,15 @@ int32_t cwbvh_scene_create_ex(const cwbvh_layout* L, void* stream, int32_t strid
         // copies queued before the failing call read host vectors freed on return
         (void)hipStreamSynchronize(st);
         if (dn) hipFree(dn);
+        if (ds) hipFree(ds);
         if (dw) hipFree(dw);
         if (dp) hipFree(dp);
         delete s;
         return hip_fail(e, "scene upload");
     }
     s->nodes = dn;
+    s->spread_nodes = ds;
+    s->spread_bytes = (int64_t)sb;
     s->woop = dw;
     s->prim_idx = (const int32_t*)dp;
     s->bytes = (int64_t)(nb + wb + pb);
@@ -399,7 +415,7 @@ int32_t cwbvh_scene_wrap_device(int32_t kind, int32_t node_stride, const void* d
 
 int32_t cwbvh_scene_device_bytes(const cwbvh_scene* s, int64_t* bytes) {
     CW_CHECK_ARG(s != nullptr && bytes != nullptr, "NULL argument");
-    *bytes = s->bytes;
+    *bytes = s->bytes + s->spread_bytes;
     return CWBVH_OK;
 }
 
@@ -419,6 +435,7 @@ void cwbvh_scene_destroy(cwbvh_scene* s) {
     if (!s) return;
     if (s->owning) {
         hipFree(const_cast<void*>(s->nodes));
+        if (s->spread_nodes) hipFree(const_cast<void*>(s->spread_nodes));
         hipFree(const_cast<void*>(s->woop));
         hipFree(const_cast<int32_t*>(s->prim_idx));
     }

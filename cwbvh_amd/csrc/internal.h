@@ -13,6 +13,11 @@ struct cwbvh_scene {
     int32_t kind = CWBVH_KIND_CWBVH;
     int32_t node_stride = 5;
     const void* nodes = nullptr;   // device
+    // Owning scenes with 128 B nodes: the same nodes with their 16-byte slots
+    // exchanged by the node's index (slot s of node i at s XOR (i mod 8)), the
+    // form that the LDS-only kernels read.
+    const void* spread_nodes = nullptr;
+    int64_t spread_bytes = 0;
     const void* woop = nullptr;    // device
     const int32_t* prim_idx = nullptr;
     int64_t woop_f4 = 0;           // valid float4 count of the Woop array (0 = unknown)
@@ -115,6 +120,9 @@ int32_t prepare_trace(const cwbvh_scene* scene, const cwbvh_ray* d_rays, const i
                       int64_t n, uint32_t flags, const cwbvh_trace_config* cfg, uint64_t* d_counters, void* stream,
                       TraceLaunch* out);
 int32_t launch_cwbvh(const TraceLaunch& L);
+// Spread nodes are addressed with 32-bit byte offsets.
+constexpr int64_t kMaxSpreadNodes = int64_t(1) << 25;
+int32_t launch_spread_nodes(const void* nodes, int64_t num_nodes, int32_t stride, void* out, hipStream_t stream);
 int32_t launch_cwbvh_surfels(const TraceLaunch& L);
 int32_t launch_surfel_rays(const cwbvh_float4* pos, const cwbvh_float4* nrm, const float* rad, int64_t num_texels,
                            int32_t rays_per_texel, float tmin, float tmax, uint64_t seed, cwbvh_ray* out,

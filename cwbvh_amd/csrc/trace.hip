@@ -151,6 +151,7 @@ struct CwbvhParams {
     int rays_per_wave;              // persistent 0: rays given to a wave, 1..64
     int num_jobs;
     int stride;                     // float4 per node: 5 or 8
+    int spread;                     // host side: nodes are spread nodes (SPREAD kernels)
     int lds_depth;
     int chunk;
     int idle_lanes;
@@ -178,6 +179,22 @@ constexpr int kRaysFromSurfels = 1;
 
 __device__ __forceinline__ const float4* node_at(const float4* nodes, unsigned i, unsigned stride_sh) {
     return nodes + ((i << 2) + (i << stride_sh));
+}
+
+// Spread nodes (internal.h): the 128 B node's 16-byte slots exchanged by the
+// node's index.  Slot s of node i sits at slot s XOR (i mod 8).  A load
+// instruction of 64 lanes reads one slot of 64 nodes; at a 128 B stride all of
+// them would sit in the same 16-byte column of their cache lines, and the L1
+// serves such a load in 64 cycles, against 34 when the columns differ
+// (measured with the lines in L1).
+__device__ __forceinline__ unsigned spread_offset(unsigned i) { return (i << 7) | ((i & 7u) << 4); }
+
+__device__ __forceinline__ const char* spread_at(const float4* nodes, unsigned offset, unsigned byte) {
+    return reinterpret_cast<const char*>(nodes) + (offset ^ byte);
+}
+
+__device__ __forceinline__ float4 spread_slot(const float4* nodes, unsigned offset, unsigned slot) {
+    return *reinterpret_cast<const float4*>(spread_at(nodes, offset, slot << 4));
 }
 
 // Quantized slab test of 4 children (one meta dword, one byte per child).
@@ -361,7 +378,7 @@ __device__ __forceinline__ void write_hit(const CwbvhParams& P, const RayState& 
 // schedule, so the hits are too: a triangle group's closest hit is its lowest
 // (t, address) under the same tie rule, its any hit the accepted triangle with
 // the highest bit.  The stack stays in the LDS column of the ray's first lane.
-template <bool ANY, int SRC, bool MULTI, int TEAM>
+template <bool ANY, int SRC, bool MULTI, bool SPREAD, int TEAM>
 __device__ __forceinline__ unsigned long long team_trace(const CwbvhParams& P, CWD_LDS unsigned long long* lds_stack,
                                                          unsigned long long live, int leave, int lane, RayState& r) {
     constexpr int kChildren = 8 / TEAM;   // children per lane: j and, teams of 4, j + 4
@@ -383,19 +400,37 @@ __device__ __forceinline__ unsigned long long team_trace(const CwbvhParams& P, C
                 const int bit = 31 - __clz((int)r.ng.y);
                 const unsigned slot = (unsigned)(bit - 24) ^ r.octinv;
                 const unsigned rel = (unsigned)__popc(imask & ~(0xFFFFFFFFu << slot));
-                const float4* np = node_at(r.nodes, r.ng.x + rel, r.stride_sh);
                 // this lane's planes: bytes lo x, y, z, hi x, y, z of 8 children each
-                const unsigned char* q = reinterpret_cast<const unsigned char*>(np + 2) + j;
-                const float4 n0 = np[0], n1 = np[1];
+                float4 n0, n1;
                 unsigned near[kChildren][3], far[kChildren][3];
+                if constexpr (SPREAD) {
+                    const unsigned off = spread_offset(r.ng.x + rel);
+                    n0 = spread_slot(r.nodes, off, 0);
+                    n1 = spread_slot(r.nodes, off, 1);
+                    auto plane = [&](int at) { return *(const unsigned char*)spread_at(r.nodes, off, (unsigned)(32 + at)); };
 #pragma unroll
-                for (int c = 0; c < kChildren; ++c) {
-                    near[c][0] = q[tx + 4 * c];
-                    near[c][1] = q[8 + ty + 4 * c];
-                    near[c][2] = q[16 + tz + 4 * c];
-                    far[c][0] = q[24 - tx + 4 * c];
-                    far[c][1] = q[32 - ty + 4 * c];
-                    far[c][2] = q[40 - tz + 4 * c];
+                    for (int c = 0; c < kChildren; ++c) {
+                        near[c][0] = plane(j + tx + 4 * c);
+                        near[c][1] = plane(j + 8 + ty + 4 * c);
+                        near[c][2] = plane(j + 16 + tz + 4 * c);
+                        far[c][0] = plane(j + 24 - tx + 4 * c);
+                        far[c][1] = plane(j + 32 - ty + 4 * c);
+                        far[c][2] = plane(j + 40 - tz + 4 * c);
+                    }
+                } else {
+                    const float4* np = node_at(r.nodes, r.ng.x + rel, r.stride_sh);
+                    const unsigned char* q = reinterpret_cast<const unsigned char*>(np + 2) + j;
+                    n0 = np[0];
+                    n1 = np[1];
+#pragma unroll
+                    for (int c = 0; c < kChildren; ++c) {
+                        near[c][0] = q[tx + 4 * c];
+                        near[c][1] = q[8 + ty + 4 * c];
+                        near[c][2] = q[16 + tz + 4 * c];
+                        far[c][0] = q[24 - tx + 4 * c];
+                        far[c][1] = q[32 - ty + 4 * c];
+                        far[c][2] = q[40 - tz + 4 * c];
+                    }
                 }
                 r.ng.y &= ~(1u << bit);
                 if (r.ng.y > 0x00FFFFFFu) {
@@ -501,7 +536,7 @@ __device__ __forceinline__ unsigned long long team_trace(const CwbvhParams& P, C
 }
 
 template <bool ANY, bool STATS, bool MULTI, bool PREFETCH, int LOOP, int SRC = kRaysFromBuffer, bool W7 = false,
-          bool LDSO = false>
+          bool LDSO = false, bool SPREAD = false>
 __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhParams P) {
     static_assert(!W7 || (LOOP == kLoopInterleave && !MULTI && !STATS && !PREFETCH),
                   "the 7-wave build is made for the plain interleaved kernels only");
@@ -509,6 +544,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
     // lds_depth stack entries, so the stack lives in LDS only (interleaved
     // schedule: only node groups are pushed, one per level of the tree)
     static_assert(!LDSO || (LOOP == kLoopInterleave && !STATS), "LDS-only stacks serve the interleaved schedule");
+    static_assert(!SPREAD || (LDSO && !MULTI), "spread nodes serve the LDS-only single-scene kernels");
     // The last rays of a wave go to teams of lanes (team_trace) where the stack
     // is in LDS.  The 7-wave builds serve launches of 2^22 rays and more, whose
     // tail is 3% of their time; with team_trace their node loop spills scalars
@@ -763,8 +799,14 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
             } else {
                 const unsigned slot = (unsigned)(bit - 24) ^ octinv;
                 const unsigned rel = (unsigned)__popc(imask & ~(0xFFFFFFFFu << slot));
-                const float4* np = node_at(nodes, base + rel, stride_sh);
-                n0 = np[0]; n1 = np[1]; n2 = np[2]; n3 = np[3]; n4 = np[4];
+                if constexpr (SPREAD) {
+                    const unsigned off = spread_offset(base + rel);
+                    n0 = spread_slot(nodes, off, 0); n1 = spread_slot(nodes, off, 1); n2 = spread_slot(nodes, off, 2);
+                    n3 = spread_slot(nodes, off, 3); n4 = spread_slot(nodes, off, 4);
+                } else {
+                    const float4* np = node_at(nodes, base + rel, stride_sh);
+                    n0 = np[0]; n1 = np[1]; n2 = np[2]; n3 = np[3]; n4 = np[4];
+                }
             }
             if (STATS) ++st_nodes;
             const unsigned eb = f2u(n0.w);
@@ -801,8 +843,14 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                 const int nb = 31 - __clz((int)ng.y);
                 const unsigned nslot = (unsigned)(nb - 24) ^ octinv;
                 const unsigned nrel = (unsigned)__popc(ng.y & ~(0xFFFFFFFFu << nslot));
-                const float4* np = node_at(nodes, ng.x + nrel, stride_sh);
-                pf0 = np[0]; pf1 = np[1]; pf2 = np[2]; pf3 = np[3]; pf4 = np[4];
+                if constexpr (SPREAD) {
+                    const unsigned off = spread_offset(ng.x + nrel);
+                    pf0 = spread_slot(nodes, off, 0); pf1 = spread_slot(nodes, off, 1); pf2 = spread_slot(nodes, off, 2);
+                    pf3 = spread_slot(nodes, off, 3); pf4 = spread_slot(nodes, off, 4);
+                } else {
+                    const float4* np = node_at(nodes, ng.x + nrel, stride_sh);
+                    pf0 = np[0]; pf1 = np[1]; pf2 = np[2]; pf3 = np[3]; pf4 = np[4];
+                }
                 have_pf = true;
             }
             return make_uint2(f2u(n1.y), hitmask & 0x00FFFFFFu);
@@ -942,8 +990,8 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
         if (live != 0ull) {
             RayState r{o, d, tmin, tmax, idx, idy, idz, octinv, ng, tg, sp, sx.col, hit_addr, out_idx,
                        out_texel, hu, hv, nodes, tris, hits, prim_map, stride_sh};
-            if (__popcll(live) > 8) live = team_trace<ANY, SRC, MULTI, 4>(P, lds_stack, live, 8, lane, r);
-            team_trace<ANY, SRC, MULTI, 8>(P, lds_stack, live, 0, lane, r);
+            if (__popcll(live) > 8) live = team_trace<ANY, SRC, MULTI, SPREAD, 4>(P, lds_stack, live, 8, lane, r);
+            team_trace<ANY, SRC, MULTI, SPREAD, 8>(P, lds_stack, live, 0, lane, r);
         }
     }
     if (STATS) {
@@ -1409,11 +1457,11 @@ void set_splits(Params& p) {
 }
 
 template <bool ANY, bool STATS, bool MULTI, bool PREFETCH, int LOOP, int SRC = kRaysFromBuffer, bool W7 = false,
-          bool LDSO = false>
+          bool LDSO = false, bool SPREAD = false>
 int32_t launch_cwbvh_t(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStream_t stream) {
     const int block = cfg.block_size;
     const size_t lds = (size_t)block * (size_t)cfg.lds_depth * sizeof(unsigned long long);
-    auto kernel = cwbvh_trace<ANY, STATS, MULTI, PREFETCH, LOOP, SRC, W7, LDSO>;
+    auto kernel = cwbvh_trace<ANY, STATS, MULTI, PREFETCH, LOOP, SRC, W7, LDSO, SPREAD>;
     long long grid = cfg.grid_blocks;
     if (!MULTI && !p.persistent) {
         // Waves of the LDS-only kernels trace their last 16 rays with 4 or 8
@@ -1495,6 +1543,7 @@ int32_t dispatch_loop(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStream_t
                                               (cfg.occupancy == kOccupancyAuto && (long long)p.n >= kOccupancy7MinRays));
                 if (p.lds_only) {
                     if (w7) return launch_cwbvh_t<ANY, false, false, false, kLoopInterleave, kRaysFromBuffer, true, true>(p, cfg, st);
+                    if (p.spread) return launch_cwbvh_t<ANY, false, false, PREFETCH, kLoopInterleave, kRaysFromBuffer, false, true, true>(p, cfg, st);
                     return launch_cwbvh_t<ANY, false, false, PREFETCH, kLoopInterleave, kRaysFromBuffer, false, true>(p, cfg, st);
                 }
                 if (w7) return launch_cwbvh_t<ANY, false, false, false, kLoopInterleave, kRaysFromBuffer, true>(p, cfg, st);
@@ -1539,6 +1588,16 @@ int32_t dispatch_surfels(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStrea
         case kLoopSpeculate: return launch_cwbvh_t<ANY, STATS, false, false, kLoopSpeculate, kRaysFromSurfels>(p, cfg, st);
         default: return launch_cwbvh_t<ANY, STATS, false, false, kLoopGroup, kRaysFromSurfels>(p, cfg, st);
     }
+}
+
+// Spread nodes from 80 B or 128 B ones: one thread per 16-byte slot.
+__global__ __launch_bounds__(256) void spread_nodes_kernel(const float4* __restrict__ nodes, long long num_nodes, int stride,
+                                                           float4* __restrict__ out) {
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= num_nodes * 8) return;
+    const long long i = t >> 3;
+    const int slot = (int)(t & 7) ^ (int)(i & 7);   // the slot stored at place t mod 8 of node i
+    out[t] = slot < 5 ? nodes[i * stride + slot] : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 // One thread per ray: the unfused generator (same arithmetic as the fused one).
@@ -1624,6 +1683,16 @@ static bool lds_only(const cwbvh_scene* s, const cwbvh_trace_config& c) {
     return s->stack_need > 0 && s->stack_need <= c.lds_depth && c.lds_depth <= kStackCapacity;
 }
 
+// The spread nodes of a scene serve its LDS-only interleaved launches (no
+// counters, rays from a buffer, the build for 6 or fewer waves).
+static void choose_nodes(CwbvhParams& p, const TraceLaunch& L) {
+    const cwbvh_trace_config& c = L.cfg;
+    const bool w7 = !c.prefetch && (c.occupancy == kOccupancy7 ||
+                                    (c.occupancy == kOccupancyAuto && (long long)L.n >= kOccupancy7MinRays));
+    p.spread = p.lds_only && L.scene->spread_nodes && c.loop_mode == kLoopInterleave && !w7 && !(L.flags & CWBVH_TRACE_STATS);
+    if (p.spread) p.nodes = (const float4*)L.scene->spread_nodes;
+}
+
 int32_t launch_cwbvh(const TraceLaunch& L) {
     const cwbvh_scene* s = L.scene;
     CwbvhParams p{};
@@ -1653,7 +1722,17 @@ int32_t launch_cwbvh(const TraceLaunch& L) {
     p.persistent = L.cfg.persistent == 2 ? (L.n >= cw::kAutoPersistentRays ? 1 : 0) : L.cfg.persistent;
     p.spec_limit = cw::speculation_limit(s->stack_need);
     p.lds_only = lds_only(s, L.cfg) ? 1 : 0;
+    choose_nodes(p, L);
     return dispatch_cwbvh<false>(p, L.flags, L.cfg, L.stream);
+}
+
+int32_t launch_spread_nodes(const void* nodes, int64_t num_nodes, int32_t stride, void* out, hipStream_t stream) {
+    const long long threads = (long long)num_nodes * 8;
+    if (threads == 0) return CWBVH_OK;
+    hipLaunchKernelGGL(spread_nodes_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream,
+                       (const float4*)nodes, (long long)num_nodes, stride, (float4*)out);
+    CW_HIP(hipGetLastError());
+    return CWBVH_OK;
 }
 
 int32_t launch_cwbvh_surfels(const TraceLaunch& L) {
