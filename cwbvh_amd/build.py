@@ -30,6 +30,8 @@ HIP_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function", "-Wno-unused-result",
 ]
+# per source, with the reason in the source
+EXTRA_FLAGS = {"trace_prefetch.hip": ["-fno-slp-vectorize"]}
 CXX_FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "-pthread", "-ffp-contract=off",
     "-D__HIP_PLATFORM_AMD__", f"-I{ROCM / 'include'}", "-Wall", "-Wno-unused-function", "-Wno-unused-result",
@@ -50,7 +52,7 @@ def _run(cmd: list[str]) -> None:
 def _compile(src: Path) -> Path:
     obj = BUILD / (src.name + ".o")
     if src.suffix == ".hip":
-        cmd = [str(ROCM / "bin" / "hipcc"), *HIP_FLAGS, "-c", str(src), "-o", str(obj)]
+        cmd = [str(ROCM / "bin" / "hipcc"), *HIP_FLAGS, *EXTRA_FLAGS.get(src.name, []), "-c", str(src), "-o", str(obj)]
     else:
         cmd = ["g++", *CXX_FLAGS, "-c", str(src), "-o", str(obj)]
     _run(cmd)
