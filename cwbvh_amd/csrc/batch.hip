@@ -311,7 +311,11 @@ int32_t cwbvh_batch_create(const cwbvh_batch_item* items, int32_t count, uint32_
     if (rc) return rc;
     // the job table is planned in chunks: fix the chunk size here so that the
     // plan and the kernel use the same value
-    if (c.fetch_chunk == 0) c.fetch_chunk = kBatchChunk;
+    if (c.fetch_chunk == 0) {
+        int64_t rays = 0;
+        for (int32_t i = 0; i < count; ++i) rays += std::max<int64_t>(0, items[i].n);
+        c.fetch_chunk = batch_chunk(rays);
+    }
     auto* b = new cwbvh_batch();
     b->flags = flags;
     b->cfg = c;

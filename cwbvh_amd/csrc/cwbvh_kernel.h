@@ -80,6 +80,12 @@ __device__ __forceinline__ unsigned slice_claim(unsigned* work, int sl, unsigned
     return (unsigned)min(static_items + base, 0xFFFFFFFFull);
 }
 
+// Whether the first claims of slice sl's waves cover all its `size` items, so
+// that nothing is left to claim from its counter.
+__device__ __forceinline__ bool static_only(int sl, unsigned size, unsigned amount, unsigned block_q, unsigned block_r) {
+    return (unsigned long long)home_blocks(sl, block_q, block_r) * (blockDim.x >> 6) * amount >= size;
+}
+
 // Marks slice `sl` drained and returns the drained mask as now known: one
 // load, and an atomic only when the slice is not marked yet.
 __device__ __forceinline__ unsigned mark_drained(unsigned* work, int sl, int lane) {
@@ -131,6 +137,7 @@ struct CwbvhParams {
     int persistent;                 // 0: each wave traces rays_per_wave rays, no refill
     int rays_per_wave;              // persistent 0: rays given to a wave, 1..64
     int num_jobs;
+    int job_step;                   // batches: jobs per lane of the chunk search, ceil(num_jobs / 64)
     int stride;                     // float4 per node: 5 or 8
     int spread;                     // host side: nodes are spread nodes (SPREAD kernels)
     int lds_depth;
@@ -586,6 +593,14 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
     const unsigned first_index =
         (blockIdx.x / (unsigned)P.slices) * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
+    // Batches: lane k holds the first chunk of job k * job_step, so a claimed
+    // chunk's job is found by one ballot (job_step 1: up to 64 jobs) and a search
+    // among job_step jobs, not by log2(jobs) dependent loads per claim.
+    unsigned seg_begin = 0xFFFFFFFFu;
+    if constexpr (MULTI && kTeams) {
+        if (lane * P.job_step < P.num_jobs) seg_begin = P.jobs[lane * P.job_step].chunk_begin;
+    }
+
     while (true) {
         const bool terminated = !busy;
         unsigned long long need = __ballot(terminated);
@@ -609,18 +624,29 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                     // range, then from the others
                     bool found = false;
                     unsigned base = 0;
+                    const bool first_claim = slice_k == 0 && pool_end == 0u;
+                    unsigned drained = 0;
                     while (slice_k < P.slices) {
                         const int sl = home + slice_k - (home + slice_k >= P.slices ? P.slices : 0);
+                        if (slice_k > 0 && ((drained >> sl) & 1u)) {
+                            ++slice_k;
+                            continue;
+                        }
                         const unsigned lo = slice_begin(sl, P.item_q, P.item_r);
                         const unsigned hi = slice_begin(sl + 1, P.item_q, P.item_r);
-                        unsigned claim = 0;
-                        if (lane == leader) claim = atomicAdd(&P.work[sl * kWorkStride], 1u);
-                        claim = __shfl(claim, leader);
+                        const bool static_claim = first_claim && slice_k == 0;
+                        if (!static_claim && static_only(sl, hi - lo, 1u, P.block_q, P.block_r)) {
+                            ++slice_k;
+                            continue;
+                        }
+                        const unsigned claim = slice_claim(P.work, sl, 1u, static_claim, first_index,
+                                                           P.block_q, P.block_r, lane);
                         if (claim < hi - lo) {
                             base = lo + claim;
                             found = true;
                             break;
                         }
+                        if (!static_claim) drained = mark_drained(P.work, sl, lane);
                         ++slice_k;
                     }
                     if (!found) {
@@ -629,6 +655,12 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                     }
                     // job j owns chunks [jobs[j].chunk_begin, jobs[j+1].chunk_begin)
                     int lo = 0, hi = P.num_jobs - 1;
+                    if constexpr (kTeams) {
+                        // all 64 lanes are here: the segment whose first job starts at or before the chunk
+                        const int seg = __popcll(__ballot(seg_begin <= base)) - 1;
+                        lo = seg * P.job_step;
+                        hi = min(lo + P.job_step, P.num_jobs) - 1;
+                    }
                     while (lo < hi) {
                         const int mid = (lo + hi + 1) >> 1;
                         if (P.jobs[mid].chunk_begin <= base) lo = mid;
@@ -988,18 +1020,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
     }
     // one-ray-per-thread launches claim nothing and skip the exit count
     if (!MULTI && !P.persistent) return;
-    if constexpr (MULTI) {
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const unsigned prev = atomicAdd(&P.work[kWorkExited], 1u);
-            if (prev == (unsigned)P.total_blocks - 1u) {
-                for (int k = 0; k < kWorkSlices; ++k) atomicExch(&P.work[k * kWorkStride], 0u);
-                atomicExch(&P.work[kWorkExited], 0u);
-            }
-        }
-    } else {
-        block_exit(P.work, P.total_blocks, P.slices, P.block_q, P.block_r);
-    }
+    block_exit(P.work, P.total_blocks, P.slices, P.block_q, P.block_r);
 }
 
 // ------------------------------------------------------------ occupancy
@@ -1061,6 +1082,12 @@ int32_t launch_cwbvh_t(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStream_
         grid = (long long)resident_blocks(kernel, block, lds) * cw::device_compute_units();
     }
     p.total_waves = (int)(grid * (block / 64));
+    if (MULTI && cfg.grid_blocks <= 0) {
+        // a batch of fewer chunks than waves: one chunk per wave, no idle blocks
+        const long long slices = std::max(1, p.slices), waves = block / 64;
+        const long long per_slice = ((long long)p.n + slices - 1) / slices;
+        grid = std::min(grid, slices * ((per_slice + waves - 1) / waves));
+    }
     p.total_blocks = (int)grid;
     set_splits(p);
     if (p.chunk <= 0) {

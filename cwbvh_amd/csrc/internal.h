@@ -166,10 +166,10 @@ struct BatchLaunch {
     hipStream_t stream;
     int32_t lds_only;         // every job's tree needs at most cfg.lds_depth stack entries
 };
-// Rays per job chunk of a multi-scene launch when the configuration asks for
-// an automatic chunk size (fetch_chunk == 0); batch plans and the kernel must
-// agree on it.
-constexpr int32_t kBatchChunk = 256;
+// Rays per job chunk of a multi-scene launch of total_rays when the
+// configuration asks for an automatic chunk size (fetch_chunk == 0); batch
+// plans and the kernel must agree on it.
+int32_t batch_chunk(int64_t total_rays);
 int32_t launch_cwbvh_batch(const BatchLaunch& L);
 
 int32_t validate_config(int32_t kind, const cwbvh_trace_config& c);

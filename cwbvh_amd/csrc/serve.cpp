@@ -168,6 +168,7 @@ struct cwbvh_server {
     int32_t launch(Slot& sl, const std::vector<Request*>& batch);
     void complete(Slot& sl);
     void fail_pending();
+    bool hold_launch() const;
     void loop();
 };
 
@@ -219,7 +220,10 @@ int32_t cwbvh_server::launch(Slot& sl, const std::vector<Request*>& batch) {
         sl.busy = true;
         return CWBVH_OK;
     }
-    const int32_t chunk = cfg.trace.fetch_chunk;
+    // each launch is planned in chunks of its own size (fetch_chunk 0: by its rays)
+    int64_t launch_rays = 0;
+    for (const Request* r : batch) launch_rays += r->n;
+    const int32_t chunk = cfg.trace.fetch_chunk > 0 ? cfg.trace.fetch_chunk : batch_chunk(launch_rays);
     uint32_t chunks = 0;
     int32_t max_need = 0;  // deepest stack need of the launch's trees (-1: unknown)
     for (size_t k = 0; k < batch.size(); ++k) {
@@ -270,6 +274,7 @@ int32_t cwbvh_server::launch(Slot& sl, const std::vector<Request*>& batch) {
         L.total_chunks = chunks;
         L.flags = cfg.flags;
         L.cfg = cfg.trace;
+        L.cfg.fetch_chunk = chunk;
         L.cfg.lds_depth = launch_lds_depth(cfg.trace.lds_depth, max_need);
         L.counters = sl.counters;
         L.stream = sl.stream;
@@ -320,6 +325,26 @@ void cwbvh_server::fail_pending() {
     pending.clear();
 }
 
+// Rays that give every SIMD of the device 4 full waves.
+static int64_t filling_rays() { return 64ll * 16 * device_compute_units(); }
+
+// Whether the pending requests wait for the launches in flight (called with
+// `mu` held).  Ray requests that do not fill the device join one launch once
+// the device is free instead of taking slots one by one: launches of a few
+// requests each would mostly pay their own start, end and copies.
+bool cwbvh_server::hold_launch() const {
+    if (cfg.serial || inflight == 0 || pending.empty()) return false;
+    const int64_t enough = std::min(filling_rays(), cfg.max_batch_rays);
+    int64_t rays = 0;
+    int32_t count = 0;
+    for (const Request* r : pending) {
+        if (r->kind == CWBVH_REQUEST_SURFELS) return false;   // a launch of its own
+        rays += r->n;
+        if (rays >= enough || ++count >= cfg.max_batch_requests) return false;
+    }
+    return true;
+}
+
 void cwbvh_server::loop() {
     std::vector<Request*> batch;
     while (true) {
@@ -358,7 +383,7 @@ void cwbvh_server::loop() {
         {
             std::unique_lock<std::mutex> lk(mu);
             if (stop && pending.empty() && inflight == 0) break;
-            if (free_slot && worker_status == CWBVH_OK) {
+            if (free_slot && worker_status == CWBVH_OK && !hold_launch()) {
                 const int32_t max_req = cfg.serial ? 1 : cfg.max_batch_requests;
                 int64_t rays = 0;
                 while (!pending.empty() && (int32_t)batch.size() < max_req) {
@@ -466,8 +491,6 @@ int32_t cwbvh_server_create(const cwbvh_scene* const* scenes, int32_t num_scenes
         CW_CHECK_ARG(scenes[i] && scenes[i]->kind == CWBVH_KIND_CWBVH &&
                          (!(c.flags & CWBVH_TRACE_PRIM_ID) || scenes[i]->prim_idx),
                      "server scenes must be CWBVH scenes");
-    if (c.trace.fetch_chunk == 0) c.trace.fetch_chunk = kBatchChunk;  // batches are planned in chunks
-    CW_CHECK_ARG(num_scenes <= CWBVH_SERVER_MAX_SCENES, "too many scenes");
     auto* s = new cwbvh_server();
     s->scenes.reserve(CWBVH_SERVER_MAX_SCENES);
     s->scenes.assign(scenes, scenes + num_scenes);

@@ -715,6 +715,21 @@ int32_t launch_surfel_rays(const cwbvh_float4* pos, const cwbvh_float4* nrm, con
     return CWBVH_OK;
 }
 
+// About 4 claims per resident wave (5 per SIMD), 64 to 256 rays each: fewer
+// leave the waves unevenly loaded at the end, more cost claims (MI355X, us at
+// 64 / 128 / 192 / 256 rays: 136 k rays in 12 jobs 94 / 113 / 133 / 150; 4.6 M
+// rays in 40 jobs 410 / 378 / 389 / 395, and 348 / 326 / 321 / 323 with batches of
+// other streams overlapping; 27 M rays in 32 jobs 2139 / 1882 / 1823 / 1815).
+// Launches that give each wave one chunk of 8 or 16 rays, traced by teams of
+// lanes from the start, do so up to 4 waves per SIMD, as single-scene launches do.
+int32_t batch_chunk(int64_t total_rays) {
+    const int64_t simds = 4ll * device_compute_units();
+    if (total_rays <= 8 * 4 * simds) return 8;
+    if (total_rays <= 16 * 4 * simds) return 16;
+    const int64_t c = total_rays / (5 * simds * 4) / 64 * 64;
+    return (int32_t)std::min<int64_t>(256, std::max<int64_t>(64, c));
+}
+
 int32_t launch_cwbvh_batch(const BatchLaunch& L) {
     if (L.cfg.fetch_chunk <= 0) {
         set_error("batch launch needs the chunk size its job table was planned with");
@@ -723,6 +738,7 @@ int32_t launch_cwbvh_batch(const BatchLaunch& L) {
     CwbvhParams p{};
     p.jobs = L.d_jobs;
     p.num_jobs = L.num_jobs;
+    p.job_step = (L.num_jobs + 63) / 64;
     p.n = (int)L.total_chunks;
     p.work = L.counters;
     p.stats = (unsigned long long*)L.stats;
