@@ -238,18 +238,34 @@ __device__ __forceinline__ unsigned child_hits4(unsigned meta4, unsigned lox, un
 //    refused by validate_config: its first GPU run faulted the device
 //    together with another untested path, and the cause was not shown, so the
 //    schedule was taken out.
-//  kLoopInterleave with the stack in LDS only (LDSO kernels): a lane holds up
-//    to two triangle groups, so it visits its next node while a first group
-//    waits its turn; the second group needs no stack room.  Triangles are tested
-//    in the order they were found, so any hits are those of the other order,
-//    and closest hits do not depend on it.  A lane with a long group then stalls
-//    less: 33 M AO rays closest hit 2.12 -> 2.03 ms, any hit 1.92 -> 1.84 ms;
-//    1 M AO rays on a heightfield 147 -> 135 us; 1920x1080 camera rays 332 -> 306
-//    us.  Holding the triangle step back until kTriangleLanes lanes hold
-//    triangles pays only for the prefetch kernels, whose scenes have the most
-//    triangle tests per visit (5 M-triangle soup: 10.83 ms at 8 lanes, 11.10 at
-//    1, 11.54 at 24; 33 M AO rays: 2.06 ms at 8, 2.05 at 1, 2.16 at 24).
+//  kLoopInterleave with the stack in LDS only (LDSO) lets a lane with a long triangle group stall less, in one of
+//    three ways; all keep each ray's sequence of visits and tests, so hits are
+//    those of kLoopGroup to the bit, ties included:
+//    - any hit (kTwoGroups): a lane holds up to two triangle groups, so it
+//      visits its next node while the first group waits.  Until its first
+//      accepted triangle an any-hit ray's interval is constant, so a visit made
+//      early finds what it would find later, and the groups are tested in the
+//      order they were found.  33 M AO rays 1.92 -> 1.84 ms.
+//    - closest hit, prefetch kernels (kLookAhead): one visit ahead, undone and
+//      made again when the waiting group shortens the ray.  Node loads bound
+//      these kernels, and a lane that waits has none in flight.  5 M-triangle
+//      soup, 16.8 M rays: 11.18 -> 11.00 ms.  (Elsewhere a visit made twice
+//      costs more than the wait: 33 M AO rays 2.11 -> 2.24 ms, batch 325 -> 358
+//      us.  Not undone, visits ahead gave 2.03 ms, but a grazing ray whose
+//      triangles tie could then report another one than in the other schedules,
+//      depending on the rays it shares a wave with.)
+//    - closest hit otherwise (kRepeatTriangles): the triangle step repeats while
+//      kTriangleAgain lanes hold triangles.  1 M AO rays on a heightfield 146 us
+//      without, 139.6 at 12 lanes, 139.7 at 9, 143 at 6, 154 at 3; 1920x1080
+//      camera rays 332 / 328 / 329 / 336 / 356; 33 M AO rays 2.15 / 2.15 / 2.16
+//      / 2.19 / 2.33 ms.
+//    The prefetch kernels, whose scenes have the most triangle tests per visit,
+//    also hold the triangle step back until kTriangleLanes lanes hold triangles
+//    (with two groups, 5 M-triangle soup: 10.83 ms at 8 lanes, 11.10 at 1, 11.54
+//    at 24; at 4 with look-ahead 1.6% slower than at 8).  The others do not (33 M
+//    AO rays: 2.06 ms at 8, 2.05 at 1, 2.16 at 24).
 constexpr int kTriangleLanes = 8;
+constexpr int kTriangleAgain = 12;
 constexpr int kLoopGroup = 0;
 constexpr int kLoopInterleave = 1;
 constexpr int kLoopSpeculate = 2;
@@ -379,8 +395,12 @@ __device__ __forceinline__ void write_hit(const CwbvhParams& P, const RayState& 
 // schedule, so the hits are too: a triangle group's closest hit is its lowest
 // (t, address) under the same tie rule, its any hit the accepted triangle with
 // the highest bit.  The stack stays in the LDS column of the ray's first lane.
-template <bool ANY, int SRC, bool MULTI, bool SPREAD, int TEAM>
+// Entries beyond lds_depth (two-level stacks) go to every lane's own `spill`:
+// the lanes of a team push and pop alike, so each holds the same copy.  Rays
+// come in and leave with none there.
+template <bool ANY, int SRC, bool MULTI, bool LDSO, bool SPREAD, int TEAM>
 __device__ __forceinline__ unsigned long long team_trace(const CwbvhParams& P, CWD_LDS unsigned long long* lds_stack,
+                                                         unsigned long long (&spill)[kStackCapacity],
                                                          unsigned long long live, int leave, int lane, RayState& r) {
     constexpr int kChildren = 8 / TEAM;   // children per lane: j and, teams of 4, j + 4
     const int team = (int)((unsigned)lane / TEAM), j = (int)((unsigned)lane % TEAM);
@@ -435,8 +455,9 @@ __device__ __forceinline__ unsigned long long team_trace(const CwbvhParams& P, C
                 }
                 r.ng.y &= ~(1u << bit);
                 if (r.ng.y > 0x00FFFFFFu) {
-                    if (r.sp < P.lds_depth) {
-                        lds_stack[(r.sp << 6) + r.col] = pack2(r.ng);
+                    if (r.sp < (LDSO ? P.lds_depth : kStackCapacity)) {
+                        if (LDSO || r.sp < P.lds_depth) lds_stack[(r.sp << 6) + r.col] = pack2(r.ng);
+                        else spill[r.sp - P.lds_depth] = pack2(r.ng);
                         ++r.sp;
                     } else {
                         P.work[kWorkOverflow] = 1u;
@@ -524,7 +545,8 @@ __device__ __forceinline__ unsigned long long team_trace(const CwbvhParams& P, C
             if (!finished && r.ng.y <= 0x00FFFFFFu) {
                 if (r.sp > 0) {
                     --r.sp;
-                    r.ng = unpack2(lds_stack[(r.sp << 6) + r.col]);
+                    if (LDSO || r.sp < P.lds_depth) r.ng = unpack2(lds_stack[(r.sp << 6) + r.col]);
+                    else r.ng = unpack2(spill[r.sp - P.lds_depth]);
                 } else {
                     finished = true;
                 }
@@ -534,7 +556,7 @@ __device__ __forceinline__ unsigned long long team_trace(const CwbvhParams& P, C
                 busy = false;
                 break;
             }
-            if (__popcll(__ballot(j == 0)) <= leave) break;
+            if (__popcll(__ballot(j == 0)) <= leave && (LDSO || !__any(r.sp > P.lds_depth))) break;
         }
     }
     return __ballot(busy && j == 0);
@@ -554,6 +576,9 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
     // is in LDS.  The 7-wave builds serve launches of 2^22 rays and more, whose
     // tail is 3% of their time; with team_trace their node loop spills scalars
     // and they run 2.3% slower (33 M AO rays: 2.19 against 2.14 ms).
+    constexpr bool kTwoGroups = ANY && LDSO;
+    constexpr bool kRepeatTriangles = !ANY && !PREFETCH && LDSO;
+    constexpr bool kLookAhead = !ANY && PREFETCH && LDSO;
     constexpr bool kTeams = LDSO && !W7;
     extern __shared__ unsigned long long lds_stack_raw[];
     CWD_LDS unsigned long long* lds_stack = lds_ptr(lds_stack_raw);
@@ -574,8 +599,10 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
     int spec_limit = P.spec_limit;
     float3 o = make_float3(0.f, 0.f, 0.f), d = o;
     float tmin = 0.f, tmax = 0.f, idx = 0.f, idy = 0.f, idz = 0.f;
-    unsigned octinv = 0, octinv4 = 0;
-    uint2 ng = make_uint2(0u, 0u), tg = make_uint2(0u, 0u), tg2 = tg;
+    unsigned octinv4 = 0;   // 7 - octant in every byte
+    // tg2.x with kLookAhead: kNoGroup unless a node was visited while tg waits
+    constexpr unsigned kNoGroup = kLookAhead ? 0xFFFFFFFFu : 0u;
+    uint2 ng = make_uint2(0u, 0u), tg = make_uint2(0u, 0u), tg2 = make_uint2(kNoGroup, 0u);
     int sp = 0;
     int hit_addr = -1;
     float hu = 0.f, hv = 0.f;
@@ -773,11 +800,10 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
             }
             safe_rcp3(d, idx, idy, idz);
             const unsigned oct = ((d.x < 0.f ? 1u : 0u) << 2) | ((d.y < 0.f ? 1u : 0u) << 1) | (d.z < 0.f ? 1u : 0u);
-            octinv = 7u - oct;
-            octinv4 = octinv * 0x01010101u;
+            octinv4 = (7u - oct) * 0x01010101u;
             ng = make_uint2(0u, 0x80000000u);
             tg = make_uint2(0u, 0u);
-            tg2 = tg;
+            tg2 = make_uint2(kNoGroup, 0u);
             sp = 0;
             hit_addr = -1;
             hu = hv = 0.f;
@@ -786,7 +812,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
         }
 
         if constexpr (kTeams) {
-            if (exhausted && __popcll(__ballot(busy)) <= kLastRays) break;
+            if (exhausted && __popcll(__ballot(busy)) <= kLastRays && (LDSO || !__any(busy && sp > P.lds_depth))) break;
             if (!busy) continue;  // idle until the wave ends
         } else {
             if (terminated && !got) break;  // no work left for this lane
@@ -816,26 +842,28 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
         };
         // Visit the highest-priority child of ng: the remainder of ng goes on
         // the stack, ng becomes the child's inner children, the child's leaf
-        // triangles are returned.
-        auto visit_node = [&]() -> uint2 {
+        // triangles are returned.  A visit ahead leaves the child, as a group of
+        // its own, in the free slot above the stack's top.
+        auto visit_node = [&](bool ahead = false) -> uint2 {
             const unsigned imask = ng.y;
             const int bit = 31 - __clz((int)ng.y);
             const unsigned base = ng.x;
             ng.y &= ~(1u << bit);
             if (ng.y > 0x00FFFFFFu) push(ng);
+            const unsigned slot = (unsigned)(bit - 24) ^ (octinv4 & 7u);
+            const unsigned visited = base + (unsigned)__popc(imask & ~(0xFFFFFFFFu << slot));
+            if (ahead) lds_stack[(sp << 6) + sx.col] = pack2(make_uint2(visited, 0x80000000u));
             float4 n0, n1, n2, n3, n4;
             if (PREFETCH && have_pf) {
                 n0 = pf0; n1 = pf1; n2 = pf2; n3 = pf3; n4 = pf4;
                 have_pf = false;
             } else {
-                const unsigned slot = (unsigned)(bit - 24) ^ octinv;
-                const unsigned rel = (unsigned)__popc(imask & ~(0xFFFFFFFFu << slot));
                 if constexpr (SPREAD) {
-                    const unsigned off = spread_offset(base + rel);
+                    const unsigned off = spread_offset(visited);
                     n0 = spread_slot(nodes, off, 0); n1 = spread_slot(nodes, off, 1); n2 = spread_slot(nodes, off, 2);
                     n3 = spread_slot(nodes, off, 3); n4 = spread_slot(nodes, off, 4);
                 } else {
-                    const float4* np = node_at(nodes, base + rel, stride_sh);
+                    const float4* np = node_at(nodes, visited, stride_sh);
                     n0 = np[0]; n1 = np[1]; n2 = np[2]; n3 = np[3]; n4 = np[4];
                 }
             }
@@ -872,7 +900,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                 // the next node visit takes the highest hit child: start its
                 // loads now so they overlap the triangle tests in between
                 const int nb = 31 - __clz((int)ng.y);
-                const unsigned nslot = (unsigned)(nb - 24) ^ octinv;
+                const unsigned nslot = (unsigned)(nb - 24) ^ (octinv4 & 7u);
                 const unsigned nrel = (unsigned)__popc(ng.y & ~(0xFFFFFFFFu << nslot));
                 if constexpr (SPREAD) {
                     const unsigned off = spread_offset(ng.x + nrel);
@@ -886,7 +914,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
             }
             return make_uint2(f2u(n1.y), hitmask & 0x00FFFFFFu);
         };
-        // Test the highest triangle of tg; true when an any-hit query is done.
+        // Test the highest triangle of tg; true when it is accepted.
         auto test_triangle = [&]() -> bool {
             const int ti = 31 - __clz((int)tg.y);
             const int addr = (int)(tg.x * 3u + (unsigned)ti * 3u);
@@ -899,7 +927,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                 hit_addr = addr;
                 hu = u;
                 hv = v;
-                return ANY;
+                return true;
             }
             return false;
         };
@@ -928,7 +956,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                         }
                     }
                     prof(true, pr_tr, pr_tru);
-                    if (test_triangle()) {
+                    if (test_triangle() && ANY) {
                         finished = true;
                         break;
                     }
@@ -942,9 +970,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                     }
                 }
             } else {
-                if constexpr (LDSO) {
-                    // a lane may hold two triangle groups, so it visits the next
-                    // node while the first group waits for the triangle step
+                if constexpr (kTwoGroups) {
                     if (tg2.y == 0u && ng.y > 0x00FFFFFFu) {
                         const uint2 ntg = visit_node();
                         if (tg.y == 0u) tg = ntg;
@@ -967,6 +993,35 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                         }
                     }
                     if (tg.y == 0u && ng.y <= 0x00FFFFFFu) finished = true;
+                } else if constexpr (kLookAhead) {
+                    auto can_visit = [&]() {
+                        return ng.y > 0x00FFFFFFu && (tg.y == 0u || (tg2.x == kNoGroup && sp + 1 < P.lds_depth));
+                    };
+                    if (can_visit()) {
+                        const uint2 ntg = visit_node(tg.y != 0u);
+                        if (tg.y == 0u) tg = ntg;
+                        else tg2 = ntg;
+                    }
+                    const bool run_tri = __popcll(__ballot(tg.y != 0u)) >= kTriangleLanes || !__any(can_visit());
+                    if (run_tri && tg.y != 0u) {
+                        if (test_triangle() && tg2.x != kNoGroup) {
+                            ng = unpack2(lds_stack[(sp << 6) + sx.col]);
+                            tg2 = make_uint2(kNoGroup, 0u);
+                            have_pf = false;
+                        }
+                        if (tg.y == 0u) {
+                            tg = tg2;
+                            tg2 = make_uint2(kNoGroup, 0u);
+                        }
+                    }
+                    if (ng.y <= 0x00FFFFFFu && tg2.x == kNoGroup) {
+                        if (sp > 0) {
+                            --sp;
+                            ng = unpack2(stack_at(sp));
+                        } else if (tg.y == 0u) {
+                            finished = true;
+                        }
+                    }
                 } else {
                     // node step: lanes without triangles (and, speculating, every
                     // lane with inner children left) visit one node
@@ -992,7 +1047,13 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                         run_tri = !__any(can_visit) || stuck * 100 >= P.postpone_pct * __popcll(__ballot(1));
                     }
                     prof(run_tri && tg.y != 0u, pr_tr, pr_tru);
-                    if (run_tri && tg.y != 0u) finished = test_triangle();
+                    if constexpr (kRepeatTriangles) {
+                        do {
+                            if (tg.y != 0u) test_triangle();
+                        } while (__popcll(__ballot(tg.y != 0u)) >= kTriangleAgain);
+                    } else {
+                        if (run_tri && tg.y != 0u) finished = test_triangle() && ANY;
+                    }
                     // out of inner children: take the next group off the stack
                     if (!finished && ng.y <= 0x00FFFFFFu) {
                         if (tg.y == 0u) {
@@ -1028,7 +1089,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                 sp = 0;
                 ng = make_uint2(0u, 0u);
                 tg = make_uint2(0u, 0u);
-                tg2 = tg;
+                tg2 = make_uint2(kNoGroup, 0u);
                 have_pf = false;
                 busy = false;
                 break;
@@ -1047,10 +1108,14 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
         // the last rays of the wave, with teams of lanes
         unsigned long long live = __ballot(busy);
         if (live != 0ull) {
-            RayState r{o, d, tmin, tmax, idx, idy, idz, octinv, ng, tg, tg2, sp, sx.col, hit_addr, out_idx,
+            if (kLookAhead && tg2.x != kNoGroup) {   // teams do not look ahead
+                ng = unpack2(lds_stack[(sp << 6) + sx.col]);
+                tg2.y = 0u;
+            }
+            RayState r{o, d, tmin, tmax, idx, idy, idz, octinv4 & 7u, ng, tg, tg2, sp, sx.col, hit_addr, out_idx,
                        out_texel, hu, hv, nodes, tris, hits, prim_map, stride_sh};
-            if (__popcll(live) > 8) live = team_trace<ANY, SRC, MULTI, SPREAD, 4>(P, lds_stack, live, 8, lane, r);
-            team_trace<ANY, SRC, MULTI, SPREAD, 8>(P, lds_stack, live, 0, lane, r);
+            if (__popcll(live) > 8) live = team_trace<ANY, SRC, MULTI, LDSO, SPREAD, 4>(P, lds_stack, spill, live, 8, lane, r);
+            team_trace<ANY, SRC, MULTI, LDSO, SPREAD, 8>(P, lds_stack, spill, live, 0, lane, r);
         }
     }
     if (STATS) {
