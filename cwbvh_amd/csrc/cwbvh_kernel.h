@@ -238,7 +238,7 @@ __device__ __forceinline__ unsigned child_hits4(unsigned meta4, unsigned lox, un
 //    refused by validate_config: its first GPU run faulted the device
 //    together with another untested path, and the cause was not shown, so the
 //    schedule was taken out.
-//  kLoopInterleave with the stack in LDS only (LDSO) lets a lane with a long triangle group stall less, in one of
+//  kLoopInterleave lets a lane with a long triangle group stall less, in one of
 //    three ways; all keep each ray's sequence of visits and tests, so hits are
 //    those of kLoopGroup to the bit, ties included:
 //    - any hit (kTwoGroups): a lane holds up to two triangle groups, so it
@@ -290,7 +290,7 @@ constexpr int kOccupancy7 = 7;
 constexpr long long kOccupancy7MinRays = 1ll << 22;  // automatic choice: launches this large
 
 #ifndef CWBVH_TRACE_ATTR
-#define CWBVH_TRACE_ATTR __attribute__((amdgpu_waves_per_eu(W7 ? 7 : (LDSO && !MULTI && !PREFETCH && SRC == 0) ? 6 : 1)))
+#define CWBVH_TRACE_ATTR __attribute__((amdgpu_waves_per_eu(W7 ? 7 : LOOP == kLoopInterleave && !STATS && !PREFETCH && SRC == 0 && !MULTI ? 6 : 1)))
 #endif
 
 // A wave whose pool is dry traces its last kLastRays rays with teams of lanes
@@ -576,10 +576,10 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
     // is in LDS.  The 7-wave builds serve launches of 2^22 rays and more, whose
     // tail is 3% of their time; with team_trace their node loop spills scalars
     // and they run 2.3% slower (33 M AO rays: 2.19 against 2.14 ms).
-    constexpr bool kTwoGroups = ANY && LDSO;
-    constexpr bool kRepeatTriangles = !ANY && !PREFETCH && LDSO;
-    constexpr bool kLookAhead = !ANY && PREFETCH && LDSO;
-    constexpr bool kTeams = LDSO && !W7;
+    constexpr bool kTwoGroups = ANY && LOOP == kLoopInterleave && !STATS;
+    constexpr bool kRepeatTriangles = !ANY && !PREFETCH && LOOP == kLoopInterleave && !STATS;
+    constexpr bool kLookAhead = !ANY && PREFETCH && LOOP == kLoopInterleave && !STATS;
+    constexpr bool kTeams = LOOP == kLoopInterleave && !STATS && !W7;
     extern __shared__ unsigned long long lds_stack_raw[];
     CWD_LDS unsigned long long* lds_stack = lds_ptr(lds_stack_raw);
     unsigned long long spill[kStackCapacity];
@@ -1181,7 +1181,7 @@ int32_t launch_cwbvh_t(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStream_
         // rays 37 / 32 / 21; 32,000 rays 36 / 32 / 28; 48,000 rays 35 / 32 / 43;
         // 96,000 rays 40 / 69 / 63)
         p.rays_per_wave = 64;
-        if (LDSO && !W7) {
+        if (LOOP == kLoopInterleave && !STATS && !W7) {
             const long long waves = 16ll * cw::device_compute_units();
             if ((p.n + 7) / 8 <= waves) p.rays_per_wave = 8;
             else if ((p.n + 15) / 16 <= waves) p.rays_per_wave = 16;
