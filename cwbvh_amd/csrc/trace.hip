@@ -16,7 +16,7 @@
 //        no check).
 //    One template serves a single scene (uniform scene pointers) and the
 //    multi-scene batch (per-lane scene pointers from a job table).
-//  * bvh2_trace: one thread per ray, Aila-Laine while-while traversal with one
+//  * bvh2_trace: one lane per ray, Aila-Laine while-while traversal with one
 //    postponed leaf and a wave-wide "any lane wants nodes" exit, Woop leaves
 //    closed by a 0x80000000 terminator (src/TraversalKernelBVH2.cu:26-178).
 //
@@ -60,6 +60,7 @@ struct Bvh2Params {
     int lds_depth;
     int woop_last;   // last valid float4 index of tris (loads past a leaf terminator clamp here)
     int prim_id;
+    int share;       // bvh2_trace: rays per wave
     // persistent launches (bvh2_trace_persistent) only
     int slices;
     int chunk;
@@ -83,13 +84,19 @@ __device__ __forceinline__ bool box2(float lox, float hix, float loy, float hiy,
     return smin <= smax;
 }
 
+// Bound by its 16-byte load instructions: each takes 16 cycles of the unit's
+// address path however few lanes are on, and a third are (33 M AO rays: TA busy
+// 91%, VALU 49%).  Tried and slower or within 7%: loads shared by node visits and
+// triangle tests with refilled lanes (8.2 M rays 1.08 ms, but slower below 2 M),
+// nodes staged in LDS by four lanes each (1.28 ms).
 template <bool ANY, bool STATS>
-__global__ __launch_bounds__(kMaxBlock) void bvh2_trace(Bvh2Params P) {
+__global__ __launch_bounds__(64) void bvh2_trace(Bvh2Params P) {
     constexpr int SENTINEL = 0x76543210;
     extern __shared__ int lds_stack_raw_i[];
     CWD_LDS int* lds_stack_i = lds_ptr(lds_stack_raw_i);
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= P.n) return;
+    // one wave per block, `share` rays per wave
+    const int i = (int)blockIdx.x * P.share + (int)threadIdx.x;
+    if ((int)threadIdx.x >= P.share || i >= P.n) return;
     int spill[kBvh2StackCapacity];
     const StackIndex sx((int)threadIdx.x, P.lds_depth);
 
@@ -457,8 +464,23 @@ int32_t launch_bvh2_t(Bvh2Params& p, const cwbvh_trace_config& cfg, bool persist
     const int block = cfg.block_size;
     const size_t lds = (size_t)block * (size_t)cfg.lds_depth * sizeof(int);
     if (!persistent) {
-        const long long grid = ((long long)p.n + block - 1) / block;
-        hipLaunchKernelGGL((bvh2_trace<ANY, STATS>), dim3((unsigned)grid), dim3(block), lds, stream, p);
+        // One wave per block, whatever block_size says: the waves share nothing,
+        // and a block of several keeps the registers and LDS of those that ended
+        // until its last one ends.  1 M-triangle spheres, AO rays, closest hit, us
+        // for blocks of 256 / 128 / 64 threads: 4,000 rays 79 / 74 / 73, 150 k 118 /
+        // 110 / 107, 780 k 214 / 211 / 199, 8.2 M 1156 / 1159 / 1103.
+        // A launch too small to fill the device gives each wave fewer rays: a wave
+        // lasts as long as the visits that its rays make in turn.  The smallest
+        // share that needs at most 4 waves per SIMD, up to 16 rays (us for 64 / 16 /
+        // 8 / 4 / 1 rays per wave: 1,000 rays 44 / 40 / 35 / 35 / 29; 8,000 rays 63
+        // / 56 / 57 / 52 / 56; 32,000 rays 71 / 64 / 64 / 64 / 136; 64,000 rays 74 /
+        // 72 / 80 / 112; 100,000 rays 80 / 87, and 81 for 32)
+        const long long waves = 16ll * cw::device_compute_units();
+        p.share = 1;
+        while (p.share < 64 && ((long long)p.n + p.share - 1) / p.share > waves) p.share *= p.share < 16 ? 2 : 4;
+        const long long grid = ((long long)p.n + p.share - 1) / p.share;
+        const size_t wave_lds = (size_t)64 * (size_t)cfg.lds_depth * sizeof(int);
+        hipLaunchKernelGGL((bvh2_trace<ANY, STATS>), dim3((unsigned)grid), dim3(64), wave_lds, stream, p);
         CW_HIP(hipGetLastError());
         return CWBVH_OK;
     }
