@@ -599,7 +599,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
     int spec_limit = P.spec_limit;
     float3 o = make_float3(0.f, 0.f, 0.f), d = o;
     float tmin = 0.f, tmax = 0.f, idx = 0.f, idy = 0.f, idz = 0.f;
-    unsigned octinv4 = 0;   // 7 - octant in every byte
+    unsigned octinv = 0, octinv4 = 0;
     // tg2.x with kLookAhead: kNoGroup unless a node was visited while tg waits
     constexpr unsigned kNoGroup = kLookAhead ? 0xFFFFFFFFu : 0u;
     uint2 ng = make_uint2(0u, 0u), tg = make_uint2(0u, 0u), tg2 = make_uint2(kNoGroup, 0u);
@@ -800,7 +800,8 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
             }
             safe_rcp3(d, idx, idy, idz);
             const unsigned oct = ((d.x < 0.f ? 1u : 0u) << 2) | ((d.y < 0.f ? 1u : 0u) << 1) | (d.z < 0.f ? 1u : 0u);
-            octinv4 = (7u - oct) * 0x01010101u;
+            octinv = 7u - oct;
+            octinv4 = octinv * 0x01010101u;
             ng = make_uint2(0u, 0x80000000u);
             tg = make_uint2(0u, 0u);
             tg2 = make_uint2(kNoGroup, 0u);
@@ -850,7 +851,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
             const unsigned base = ng.x;
             ng.y &= ~(1u << bit);
             if (ng.y > 0x00FFFFFFu) push(ng);
-            const unsigned slot = (unsigned)(bit - 24) ^ (octinv4 & 7u);
+            const unsigned slot = (unsigned)(bit - 24) ^ octinv;
             const unsigned visited = base + (unsigned)__popc(imask & ~(0xFFFFFFFFu << slot));
             if (ahead) lds_stack[(sp << 6) + sx.col] = pack2(make_uint2(visited, 0x80000000u));
             float4 n0, n1, n2, n3, n4;
@@ -900,7 +901,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                 // the next node visit takes the highest hit child: start its
                 // loads now so they overlap the triangle tests in between
                 const int nb = 31 - __clz((int)ng.y);
-                const unsigned nslot = (unsigned)(nb - 24) ^ (octinv4 & 7u);
+                const unsigned nslot = (unsigned)(nb - 24) ^ octinv;
                 const unsigned nrel = (unsigned)__popc(ng.y & ~(0xFFFFFFFFu << nslot));
                 if constexpr (SPREAD) {
                     const unsigned off = spread_offset(ng.x + nrel);
@@ -1112,7 +1113,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
                 ng = unpack2(lds_stack[(sp << 6) + sx.col]);
                 tg2.y = 0u;
             }
-            RayState r{o, d, tmin, tmax, idx, idy, idz, octinv4 & 7u, ng, tg, tg2, sp, sx.col, hit_addr, out_idx,
+            RayState r{o, d, tmin, tmax, idx, idy, idz, octinv, ng, tg, tg2, sp, sx.col, hit_addr, out_idx,
                        out_texel, hu, hv, nodes, tris, hits, prim_map, stride_sh};
             if (__popcll(live) > 8) live = team_trace<ANY, SRC, MULTI, LDSO, SPREAD, 4>(P, lds_stack, spill, live, 8, lane, r);
             team_trace<ANY, SRC, MULTI, LDSO, SPREAD, 8>(P, lds_stack, spill, live, 0, lane, r);
