@@ -55,13 +55,13 @@ void bind(cwbvh_scene*& slot, int32_t kind, int32_t stride, const cwbvh_float4* 
 // the kernel with the stack in LDS only.  A tree that overflows it is traced
 // again with the two-level stack, and from then on always, until the next bind.
 // 1 M-triangle spheres, AO rays, two-level / LDS only: 4.0 M rays 540 / 491 us,
-// 1 M 178 / 160, 300 k 89 / 86.  From 2^22 rays up the 7-wave builds take over
-// (8 M: 974 / 977), and larger scenes' prefetch kernels run at 5 waves: those keep
+// 1 M 178 / 160, 300 k 89 / 86.  From 3 x 2^21 rays up the 7-wave builds take
+// over (8 M: 974 / 977), and larger scenes' prefetch kernels run at 5 waves: those keep
 // the plain launch.
 constexpr int32_t kShallowDepth = 13;
 
 bool assume_shallow(const cwbvh_scene* scene, int count, cwbvh_scene* shallow, cwbvh_trace_config* cfg) {
-    if (scene->kind != CWBVH_KIND_CWBVH || scene->stack_need > 0 || g_cwbvh_deep || count >= (1 << 22)) return false;
+    if (scene->kind != CWBVH_KIND_CWBVH || scene->stack_need > 0 || g_cwbvh_deep || count >= 3 << 21) return false;
     if (cwbvh_trace_config_for_scene(scene, cfg) != CWBVH_OK || cfg->prefetch || cfg->loop_mode != 1) return false;
     *shallow = *scene;
     shallow->stack_need = kShallowDepth;

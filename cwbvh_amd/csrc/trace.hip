@@ -524,7 +524,7 @@ int32_t dispatch_surfels(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStrea
         case kLoopInterleave:
             if constexpr (!STATS) {
                 const bool w7 = cfg.occupancy == kOccupancy7 ||
-                                (cfg.occupancy == kOccupancyAuto && (long long)p.n >= kOccupancy7MinRays);
+                                (cfg.occupancy == kOccupancyAuto && (long long)p.n >= kOccupancy7MinSurfelRays);
                 if (p.lds_only) {
                     if (w7) return launch_cwbvh_t<ANY, false, false, false, kLoopInterleave, kRaysFromSurfels, true, true>(p, cfg, st);
                     return launch_cwbvh_t<ANY, false, false, false, kLoopInterleave, kRaysFromSurfels, false, true>(p, cfg, st);
@@ -668,7 +668,8 @@ int32_t launch_cwbvh(const TraceLaunch& L) {
     // start-up and exit cost outweighs its load balancing (MI355X, AO rays on a
     // 65 k-triangle heightfield: 262 k rays trace 1.9x faster one per thread,
     // 1 M rays 15% slower)
-    p.persistent = L.cfg.persistent == 2 ? (L.n >= cw::kAutoPersistentRays ? 1 : 0) : L.cfg.persistent;
+    const int64_t pers_from = (L.flags & CWBVH_TRACE_ANY) ? cw::kAutoPersistentAnyRays : cw::kAutoPersistentRays;
+    p.persistent = L.cfg.persistent == 2 ? (L.n >= pers_from ? 1 : 0) : L.cfg.persistent;
     p.spec_limit = cw::speculation_limit(s->stack_need);
     p.lds_only = lds_only(s, L.cfg) ? 1 : 0;
     choose_nodes(p, L);
@@ -708,7 +709,7 @@ int32_t launch_cwbvh_surfels(const TraceLaunch& L) {
     p.postpone_pct = L.cfg.postpone_pct;
     p.prim_id = (L.flags & CWBVH_TRACE_PRIM_ID) ? 1 : 0;
     p.slices = L.cfg.work_slices;
-    p.persistent = L.cfg.persistent == 2 ? (L.n >= cw::kAutoPersistentRays ? 1 : 0) : L.cfg.persistent;
+    p.persistent = L.cfg.persistent == 2 ? (L.n >= cw::kAutoPersistentSurfelRays ? 1 : 0) : L.cfg.persistent;
     p.spec_limit = cw::speculation_limit(s->stack_need);
     p.lds_only = lds_only(s, L.cfg) ? 1 : 0;
     p.surf_pos = (const float4*)L.surf_pos;
