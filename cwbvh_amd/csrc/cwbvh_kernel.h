@@ -272,18 +272,17 @@ constexpr int kLoopSpeculate = 2;
 constexpr int kLoopQueue = 3;
 
 // Register budget (cwbvh_trace_config.occupancy).  The plain interleaved
-// kernel (one scene, no counters, no prefetch) takes 75 VGPRs unconstrained
-// when it reads rays from a buffer (6 waves per SIMD), 91 when it makes them
-// from surfels (5 waves).  Both are also built for 7 waves (72 VGPRs; 2 and
-// 10 registers of cold state spilled), which traces launches of tens of
-// millions of AO rays 3-5% faster and launches of a million rays 6-7% slower
-// (more waves, each slower, lengthen the tail of a short launch).  The other
-// instances stay unconstrained: the batch, counting and prefetching kernels
-// spill 10 to 32 registers at 7 waves, and the grouped and speculative
-// schedules serve scenes that stream from HBM, where spills and the extra
-// wave cost more.  The LDS-only build that reads rays from a buffer is held to
-// 6 waves: team_trace's code would lift it from 76 to 83 VGPRs, i.e. to 5; held,
-// it takes 77-79 and spills nothing.
+// kernels (one scene, no counters, no prefetch) that read rays from a buffer are
+// held to 6 waves: team_trace's code would lift them from 76 to 83 VGPRs, i.e. to
+// 5; held, they take 75-78 and spill nothing.  Those that make rays from surfels
+// take 84-89 (5 waves).  Both are also built for 7 waves (72 VGPRs; up to 1 and 6
+// registers of cold state spilled), which traces launches of tens of millions of
+// AO rays 3-5% faster and launches of a million rays 6-7% slower (more waves,
+// each slower, lengthen the tail of a short launch).  The other instances stay
+// unconstrained: the batch kernels (84-89) and the prefetch kernels (93-96, 5
+// waves) would spill 10 registers or more at 7 waves, and the grouped and
+// speculative schedules serve scenes that stream from HBM, where spills and the
+// extra wave cost more.
 constexpr int kOccupancyAuto = 0;
 constexpr int kOccupancyFree = 1;
 constexpr int kOccupancy7 = 7;
@@ -580,7 +579,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
     static_assert(!LDSO || (LOOP == kLoopInterleave && !STATS), "LDS-only stacks serve the interleaved schedule");
     static_assert(!SPREAD || (LDSO && !MULTI), "spread nodes serve the LDS-only single-scene kernels");
     // The last rays of a wave go to teams of lanes (team_trace) where the stack
-    // is in LDS.  The 7-wave builds serve launches of 2^22 rays and more, whose
+    // is in LDS.  The 7-wave builds serve launches of 3 x 2^21 rays and more, whose
     // tail is 3% of their time; with team_trace their node loop spills scalars
     // and they run 2.3% slower (33 M AO rays: 2.19 against 2.14 ms).
     constexpr bool kTwoGroups = ANY && LOOP == kLoopInterleave && !STATS;

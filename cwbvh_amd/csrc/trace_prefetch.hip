@@ -2,7 +2,7 @@
 // Infinity Cache).  They are compiled without SLP vectorization (build.py): it
 // groups the 8 children's slab tests into vector operations that keep all
 // planes in registers at once, 106 VGPRs (4 waves per SIMD) for the LDS-only
-// kernel; without it 90 (5 waves).  These launches wait on memory, so waves
+// kernel; without it 93-96 (5 waves).  These launches wait on memory, so waves
 // matter most: 5 M-triangle soup, 16.8 M shuffled rays, closest hit: 11.94 ms
 // with it, 11.40 ms without.  The kernels without prefetch keep it: they are
 // bound by instruction issue, and its grouping is 1-4% faster there (1 M AO

@@ -344,7 +344,9 @@ typedef struct cwbvh_trace_config {
     int32_t block_size;      /* 64, 128 or 256 threads (BVH2 with one ray per lane: always blocks of 64) */
     int32_t lds_depth;       /* stack entries per lane kept in LDS (1..stack capacity) */
     int32_t grid_blocks;     /* persistent grid (0 = fill the device) */
-    int32_t fetch_chunk;     /* rays claimed per wave-level atomic (persistent grids; 0 = automatic) */
+    int32_t fetch_chunk;     /* rays claimed per wave-level atomic (persistent grids; 0 = automatic: 64..512
+                                by the launch's rays per wave, 64 with a ray order, 32 with prefetch;
+                                batches 8..256) */
     int32_t refill_idle;     /* leave the inner loop once idle lanes exceed this ... */
     int32_t refill_budget;   /* ... for this many accumulated lane-iterations */
     int32_t postpone_pct;    /* 0 = off; loop_mode 0: postpone a triangle group when fewer than this %
@@ -353,20 +355,23 @@ typedef struct cwbvh_trace_config {
                                 not for loop_mode 1 */
     int32_t prefetch;        /* 0 or 1: issue the next node's loads before the triangle loop */
     int32_t work_slices;     /* 1..8 contiguous ray ranges, one drained first per XCD (persistent grids) */
-    int32_t persistent;      /* 1 = persistent grid with work fetching, 0 = one ray per thread,
-                                2 = persistent from 786,432 (3 x 2^18) rays up.  CWBVH default 2.  BVH2 default 0
-                                (the reference's kernel); its persistent grid hands rays to idle lanes
+    int32_t persistent;      /* 1 = persistent grid with work fetching, 0 = one ray per lane (launches too
+                                small to fill the device: fewer rays per wave, CWBVH 8, 16 or 64, BVH2 1 to
+                                16 or 64), 2 = persistent from 786,432 (3 x 2^18) rays up, CWBVH any hit
+                                from 1,310,720 (5 x 2^18), rays made from surfels from 2,097,152 (2^21).
+                                CWBVH default 2.  BVH2 default 0 (the reference's kernel); its persistent grid hands rays to idle lanes
                                 between while-while rounds and uses grid_blocks, fetch_chunk,
                                 refill_idle (>= 0), refill_budget (>= 1) and work_slices.  BVH2
                                 configurations keep loop_mode, prefetch, postpone_pct and occupancy 0 */
     int32_t loop_mode;       /* CWBVH inner-loop schedule: 0 = node visit + its whole triangle group
                                 per iteration (reference order), 1 = node visit or one triangle test
-                                per iteration, 2 = as 1, and lanes holding triangles also visit a
+                                per iteration (a lane with waiting triangles looks ahead where that
+                                keeps its order, see cwbvh_kernel.h), 2 = as 1, and lanes holding triangles also visit a
                                 node, parking its triangle group on the stack; 3 (per-wave triangle
                                 queue) was taken out and is refused with CWBVH_ERR_INVALID_ARGUMENT */
     int32_t occupancy;       /* register budget of the single-scene loop_mode 1 kernels (no prefetch,
                                 no stats; rays from a buffer or from surfels): 0 = automatic
-                                (7 waves per SIMD for launches of 2^22 rays or more), 1 = unconstrained,
+                                (7 waves per SIMD for launches of 3 x 2^21 rays or more, from surfels 2^22), 1 = unconstrained,
                                 7 = 7 waves per SIMD (72 VGPRs) */
     int32_t ray_order;       /* 0 = trace rays in the given order; 1 = a launch of 2^20 rays or more
                                 first sorts them by direction octant and origin Morton code (as
