@@ -1186,11 +1186,16 @@ int32_t launch_cwbvh_t(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStream_
         // waves queue behind one another (MI355X, AO rays on a 65 k-triangle
         // heightfield, closest hit, us for 64 / 16 / 8 rays per wave: 1,000
         // rays 37 / 32 / 21; 32,000 rays 36 / 32 / 28; 48,000 rays 35 / 32 / 43;
-        // 96,000 rays 40 / 69 / 63)
+        // 96,000 rays 40 / 69 / 63).  Up to half a wave per SIMD, 4 rays per wave:
+        // the teams of a wave wait for one another's loads (same scene, closest
+        // hit, us for 8 / 4 / 2 rays per wave: 500 rays 20.1 / 17.6 / 17.1, 1,000 20.4
+        // / 18.8 / 18.7, 2,000 20.3 / 20.0 / 19.7; 300 k-triangle soup, 1,000 rays 50.3 /
+        // 49.2 / 52.6, 2,000 50.1 / 48.9 / 48.4, 4,000 50.7 / 51.1 / 55.6)
         p.rays_per_wave = 64;
         if (LOOP == kLoopInterleave && !STATS && !W7) {
             const long long waves = 16ll * cw::device_compute_units();
-            if ((p.n + 7) / 8 <= waves) p.rays_per_wave = 8;
+            if ((p.n + 3) / 4 <= waves / 8) p.rays_per_wave = 4;
+            else if ((p.n + 7) / 8 <= waves) p.rays_per_wave = 8;
             else if ((p.n + 15) / 16 <= waves) p.rays_per_wave = 16;
         }
         const long long per_block = (long long)p.rays_per_wave * (block / 64);

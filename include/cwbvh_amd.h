@@ -356,7 +356,7 @@ typedef struct cwbvh_trace_config {
     int32_t prefetch;        /* 0 or 1: issue the next node's loads before the triangle loop */
     int32_t work_slices;     /* 1..8 contiguous ray ranges, one drained first per XCD (persistent grids) */
     int32_t persistent;      /* 1 = persistent grid with work fetching, 0 = one ray per lane (launches too
-                                small to fill the device: fewer rays per wave, CWBVH 8, 16 or 64, BVH2 1 to
+                                small to fill the device: fewer rays per wave, CWBVH 4, 8, 16 or 64, BVH2 1 to
                                 16 or 64), 2 = persistent from 786,432 (3 x 2^18) rays up, CWBVH any hit
                                 from 1,310,720 (5 x 2^18), rays made from surfels from 2,097,152 (2^21).
                                 CWBVH default 2.  BVH2 default 0 (the reference's kernel); its persistent grid hands rays to idle lanes

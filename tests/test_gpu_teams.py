@@ -73,3 +73,13 @@ def test_jobs_of_a_batch_share_waves(cw, scene, any_hit):
     for dr, dh, f, n, s in bufs:
         if s is sc:
             assert np.array_equal(bits(dh.download((n, 4))), refs[any_hit][f:f + n]), n
+
+
+@pytest.mark.parametrize("any_hit", [False, True])
+def test_four_rays_per_wave(cw, scene, any_hit):
+    """4 rays per wave up to 4 x 2 x 256 = 2,048 rays, then 8."""
+    sc, rays, refs = scene
+    for n in (2, 3, 4, 5, 2044, 2047, 2048, 2049, 2056):
+        print(f"[gpu-test] four per wave n={n} any={any_hit}", flush=True)
+        got = bits(sc.trace_numpy(rays[:n], cw.TRACE_ANY if any_hit else cw.TRACE_CLOSEST))
+        assert np.array_equal(got, refs[any_hit][:n]), n
