@@ -61,6 +61,7 @@ struct Bvh2Params {
     int woop_last;   // last valid float4 index of tris (loads past a leaf terminator clamp here)
     int prim_id;
     int share;       // bvh2_trace: rays per wave
+    int in_l2;       // host side: the scene fits one XCD's L2
     // persistent launches (bvh2_trace_persistent) only
     int slices;
     int chunk;
@@ -90,13 +91,14 @@ __device__ __forceinline__ bool box2(float lox, float hix, float loy, float hiy,
 // triangle tests with refilled lanes (8.2 M rays 1.08 ms, but slower below 2 M),
 // nodes staged in LDS by four lanes each (1.28 ms).
 template <bool ANY, bool STATS>
-__global__ __launch_bounds__(64) void bvh2_trace(Bvh2Params P) {
+__global__ __launch_bounds__(kMaxBlock) void bvh2_trace(Bvh2Params P) {
     constexpr int SENTINEL = 0x76543210;
     extern __shared__ int lds_stack_raw_i[];
     CWD_LDS int* lds_stack_i = lds_ptr(lds_stack_raw_i);
-    // one wave per block, `share` rays per wave
-    const int i = (int)blockIdx.x * P.share + (int)threadIdx.x;
-    if ((int)threadIdx.x >= P.share || i >= P.n) return;
+    // `share` rays per wave
+    const int slot = (int)(threadIdx.x & 63u);
+    const int i = (int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * P.share + slot;
+    if (slot >= P.share || i >= P.n) return;
     int spill[kBvh2StackCapacity];
     const StackIndex sx((int)threadIdx.x, P.lds_depth);
 
@@ -469,6 +471,12 @@ int32_t launch_bvh2_t(Bvh2Params& p, const cwbvh_trace_config& cfg, bool persist
         // until its last one ends.  1 M-triangle spheres, AO rays, closest hit, us
         // for blocks of 256 / 128 / 64 threads: 4,000 rays 79 / 74 / 73, 150 k 118 /
         // 110 / 107, 780 k 214 / 211 / 199, 8.2 M 1156 / 1159 / 1103.
+        // Not so for a million rays and more in a scene that fits one XCD's 4 MB of L2: its
+        // waves are short and end together, and dispatching them one by one costs
+        // 1-4% (heightfields, us for blocks of 256 / 64: 0.5 MB 2 M rays 236 / 241, 8 M
+        // 876 / 913; 3.1 MB 1 M 196 / 195, 2 M 357 / 361, 8 M 1298 / 1333; but 6.1 MB 2 M
+        // 445 / 431, 8 M 1631 / 1571).
+        const int one_block = p.in_l2 && p.n >= (1 << 20) ? block : 64;
         // A launch too small to fill the device gives each wave fewer rays: a wave
         // lasts as long as the visits that its rays make in turn.  The smallest
         // share that needs at most 4 waves per SIMD, up to 16 rays (us for 64 / 16 /
@@ -478,9 +486,10 @@ int32_t launch_bvh2_t(Bvh2Params& p, const cwbvh_trace_config& cfg, bool persist
         const long long waves = 16ll * cw::device_compute_units();
         p.share = 1;
         while (p.share < 64 && ((long long)p.n + p.share - 1) / p.share > waves) p.share *= p.share < 16 ? 2 : 4;
-        const long long grid = ((long long)p.n + p.share - 1) / p.share;
-        const size_t wave_lds = (size_t)64 * (size_t)cfg.lds_depth * sizeof(int);
-        hipLaunchKernelGGL((bvh2_trace<ANY, STATS>), dim3((unsigned)grid), dim3(64), wave_lds, stream, p);
+        const long long per_block = (long long)p.share * (one_block / 64);
+        const long long grid = ((long long)p.n + per_block - 1) / per_block;
+        const size_t block_lds = (size_t)one_block * (size_t)cfg.lds_depth * sizeof(int);
+        hipLaunchKernelGGL((bvh2_trace<ANY, STATS>), dim3((unsigned)grid), dim3(one_block), block_lds, stream, p);
         CW_HIP(hipGetLastError());
         return CWBVH_OK;
     }
@@ -792,6 +801,7 @@ int32_t launch_bvh2(const TraceLaunch& L) {
     p.lds_depth = L.cfg.lds_depth;
     p.woop_last = s->woop_f4 > 0 ? (int)(s->woop_f4 - 1) : 0x7FFFFFFF;
     p.prim_id = (L.flags & CWBVH_TRACE_PRIM_ID) ? 1 : 0;
+    p.in_l2 = s->bytes > 0 && s->bytes <= (4ll << 20);
     // persistent 2 = automatic: the persistent grid from kAutoPersistentRays up
     const bool pers = L.cfg.persistent == 2 ? L.n >= cw::kAutoPersistentRays : L.cfg.persistent == 1;
     const bool any = (L.flags & CWBVH_TRACE_ANY) != 0, stats = (L.flags & CWBVH_TRACE_STATS) != 0;

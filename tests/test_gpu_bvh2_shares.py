@@ -36,3 +36,19 @@ def test_every_share(cw, scene, any_hit, cfg):
         print(f"[gpu-test] bvh2 share n={n} any={any_hit} {cfg}", flush=True)
         got = bits(sc.trace_numpy(rays[:n], cw.TRACE_ANY if any_hit else cw.TRACE_CLOSEST, sc.default_config(**cfg)))
         assert np.array_equal(got, refs[any_hit][:n]), n
+
+
+@pytest.mark.parametrize("any_hit", [False, True])
+def test_blocks_of_a_scene_in_l2(cw, orc, any_hit):
+    """A scene of up to 4 MB: blocks of block_size threads from 2^20 rays up."""
+    mesh = cw.Mesh.heightfield(60, 40, 5, 0.1, seed=45)
+    lay, _ = cw.build_layouts(mesh, cwbvh=False)
+    sc = cw.Scene(lay)
+    assert sc.device_bytes() <= 4 << 20
+    n = (1 << 20) + 65
+    rays = cw.rays_ao_surface(mesh, (n + 7) // 8, 8, 1e-4 * mesh.diagonal(), 0.0, 0.1 * mesh.diagonal(), seed=46)[:n]
+    ref = bits(orc.trace_bvh2(lay.nodes, lay.woop, rays, any_hit=any_hit))
+    for m, cfg in ((n, {}), ((1 << 20) - 1, {}), (1 << 20, dict(block_size=128)), (n, dict(block_size=64, lds_depth=2))):
+        print(f"[gpu-test] bvh2 in L2 n={m} any={any_hit} {cfg}", flush=True)
+        got = bits(sc.trace_numpy(rays[:m], cw.TRACE_ANY if any_hit else cw.TRACE_CLOSEST, sc.default_config(**cfg)))
+        assert np.array_equal(got, ref[:m]), (m, cfg)
