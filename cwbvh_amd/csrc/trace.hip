@@ -476,7 +476,11 @@ int32_t launch_bvh2_t(Bvh2Params& p, const cwbvh_trace_config& cfg, bool persist
         // 1-4% (heightfields, us for blocks of 256 / 64: 0.5 MB 2 M rays 236 / 241, 8 M
         // 876 / 913; 3.1 MB 1 M 196 / 195, 2 M 357 / 361, 8 M 1298 / 1333; but 6.1 MB 2 M
         // 445 / 431, 8 M 1631 / 1571).
-        const int one_block = p.in_l2 && p.n >= (1 << 20) ? block : 64;
+        // Elsewhere what a block per wave saves at the end of a launch outweighs the
+        // dispatching until about 25 M rays (1 M-triangle spheres, any hit, us for
+        // blocks of 256 / 64: 8.2 M 1231 / 1187, 14.5 M 2139 / 2105, 20 M 2881 / 2856,
+        // 33 M 3973 / 3984).
+        const int one_block = p.n >= (p.in_l2 ? 1 << 20 : 3 << 23) ? block : 64;
         // A launch too small to fill the device gives each wave fewer rays: a wave
         // lasts as long as the visits that its rays make in turn.  The smallest
         // share that needs at most 4 waves per SIMD, up to 16 rays (us for 64 / 16 /

@@ -341,8 +341,8 @@ void cwbvh_scene_destroy(cwbvh_scene* scene);
 /* ------------------------------------------------------------ trace --- */
 
 typedef struct cwbvh_trace_config {
-    int32_t block_size;      /* 64, 128 or 256 threads (BVH2 with one ray per lane: 64, but for scenes
-                                up to 4 MB from 2^20 rays up) */
+    int32_t block_size;      /* 64, 128 or 256 threads (BVH2 with one ray per lane: 64, except from
+                                3 x 2^23 rays up, scenes up to 4 MB from 2^20) */
     int32_t lds_depth;       /* stack entries per lane kept in LDS (1..stack capacity) */
     int32_t grid_blocks;     /* persistent grid (0 = fill the device) */
     int32_t fetch_chunk;     /* rays claimed per wave-level atomic (persistent grids; 0 = automatic: 64..512
