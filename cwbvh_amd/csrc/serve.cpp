@@ -491,6 +491,7 @@ int32_t cwbvh_server_create(const cwbvh_scene* const* scenes, int32_t num_scenes
         CW_CHECK_ARG(scenes[i] && scenes[i]->kind == CWBVH_KIND_CWBVH &&
                          (!(c.flags & CWBVH_TRACE_PRIM_ID) || scenes[i]->prim_idx),
                      "server scenes must be CWBVH scenes");
+    CW_CHECK_ARG(num_scenes <= CWBVH_SERVER_MAX_SCENES, "too many scenes");
     auto* s = new cwbvh_server();
     s->scenes.reserve(CWBVH_SERVER_MAX_SCENES);
     s->scenes.assign(scenes, scenes + num_scenes);

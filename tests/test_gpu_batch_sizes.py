@@ -39,3 +39,9 @@ def test_every_plan(cw, data, jobs, total, any_hit):
         batch.launch()
     cw.synchronize()
     assert np.array_equal(bits(d_hits.download((total, 4))), refs[any_hit][:total])
+
+
+def test_server_refuses_more_scenes_than_its_table(cw, data):
+    sc = data[0]
+    with pytest.raises(cw.CwbvhError, match="too many scenes"):
+        cw.Server([sc] * 4097)
