@@ -30,8 +30,6 @@ namespace {
 std::mutex g_mu;
 cwbvh_scene* g_cwbvh = nullptr;
 cwbvh_scene* g_bvh2 = nullptr;
-// the bound CWBVH tree has overflowed kShallowDepth stack entries
-bool g_cwbvh_deep = false;
 thread_local int32_t g_status = CWBVH_OK;
 thread_local float g_ms = 0.f;
 int g_log = 1;
@@ -43,29 +41,21 @@ void bind(cwbvh_scene*& slot, int32_t kind, int32_t stride, const cwbvh_float4* 
         cwbvh_scene_destroy(slot);
         slot = nullptr;
     }
-    if (kind == CWBVH_KIND_CWBVH) g_cwbvh_deep = false;
     g_status = cwbvh_scene_wrap_device(kind, stride, nodes, woop, map, 0, &slot);
 }
 
-// Bound arrays come without the tree's stack need, so a plain trace keeps a
-// stack with a scratch part, which costs the kernel about 10%.  A bound trace
-// waits for its launch and reads the overflow flag anyway: it first assumes a
-// need of kShallowDepth entries (the deepest that leaves room for 6 waves per
-// SIMD in LDS; 8-wide trees of a million triangles need 10 or 11) and launches
-// the kernel with the stack in LDS only.  A tree that overflows it is traced
-// again with the two-level stack, and from then on always, until the next bind.
-// 1 M-triangle spheres, AO rays, two-level / LDS only: 4.0 M rays 540 / 491 us,
-// 1 M 178 / 160, 300 k 89 / 86.  From 3 x 2^21 rays up the 7-wave builds take
-// over (8 M: 974 / 977), and larger scenes' prefetch kernels run at 5 waves: those keep
-// the plain launch.
-constexpr int32_t kShallowDepth = 13;
+// Bound arrays come without the tree's stack need, so their launch keeps a stack
+// with a scratch part, and 12 entries of it in LDS: trees of a million triangles
+// need 9 to 11, and more than 12 leave room for fewer than 6 waves per SIMD.  AO
+// rays, us for 10 / 12 / 13 entries: 980 k-triangle spheres, 4.0 M rays 537 / 528
+// / 553, 1 M 179 / 176 / 191; 400 k-triangle heightfield 536 / 535 / 559, 180 / 179
+// / 201.  The 7-wave builds have room for 11 and keep the default.
+constexpr int32_t kBoundLdsDepth = 12;
 
-bool assume_shallow(const cwbvh_scene* scene, int count, cwbvh_scene* shallow, cwbvh_trace_config* cfg) {
-    if (scene->kind != CWBVH_KIND_CWBVH || scene->stack_need > 0 || g_cwbvh_deep || count >= 3 << 21) return false;
+bool bound_config(const cwbvh_scene* scene, int count, cwbvh_trace_config* cfg) {
+    if (scene->kind != CWBVH_KIND_CWBVH || count >= cw::kOccupancy7MinRays) return false;
     if (cwbvh_trace_config_for_scene(scene, cfg) != CWBVH_OK || cfg->prefetch || cfg->loop_mode != 1) return false;
-    *shallow = *scene;
-    shallow->stack_need = kShallowDepth;
-    cfg->lds_depth = kShallowDepth;
+    cfg->lds_depth = kBoundLdsDepth;
     return true;
 }
 
@@ -95,22 +85,11 @@ void trace(cwbvh_scene* scene, cwbvh_ray* rays, cwbvh_hit* hits, int count, cons
     roctxProfilerResume(0);
     roctxRangePush(label);
     hipEventRecord(a, nullptr);
-    cwbvh_scene shallow_scene;
-    cwbvh_trace_config shallow_cfg;
-    const bool shallow = assume_shallow(scene, count, &shallow_scene, &shallow_cfg);
-    int32_t rc = cwbvh_trace(shallow ? &shallow_scene : scene, rays, hits, count, CWBVH_TRACE_CLOSEST,
-                             shallow ? &shallow_cfg : nullptr, nullptr, nullptr);
+    cwbvh_trace_config cfg;
+    int32_t rc = cwbvh_trace(scene, rays, hits, count, CWBVH_TRACE_CLOSEST,
+                             bound_config(scene, count, &cfg) ? &cfg : nullptr, nullptr, nullptr);
     hipEventRecord(b, nullptr);
     hipError_t e = hipEventSynchronize(b);
-    int32_t of = 0;
-    if (rc == CWBVH_OK && e == hipSuccess) rc = cwbvh_stack_overflowed(nullptr, &of);
-    if (rc == CWBVH_OK && of && shallow) {
-        g_cwbvh_deep = true;
-        rc = cwbvh_trace(scene, rays, hits, count, CWBVH_TRACE_CLOSEST, nullptr, nullptr, nullptr);
-        hipEventRecord(b, nullptr);
-        e = hipEventSynchronize(b);
-        if (rc == CWBVH_OK && e == hipSuccess) rc = cwbvh_stack_overflowed(nullptr, &of);
-    }
     roctxRangePop();
     roctxProfilerPause(0);
     if (rc == CWBVH_OK && e != hipSuccess) rc = cw::hip_fail(e, "rtTrace");
@@ -118,9 +97,13 @@ void trace(cwbvh_scene* scene, cwbvh_ray* rays, cwbvh_hit* hits, int count, cons
     hipEventElapsedTime(&ms, a, b);
     hipEventDestroy(a);
     hipEventDestroy(b);
-    if (rc == CWBVH_OK && of) {
-        cw::set_error("traversal stack overflow");
-        rc = CWBVH_ERR_STACK_DEPTH;
+    if (rc == CWBVH_OK) {
+        int32_t of = 0;
+        rc = cwbvh_stack_overflowed(nullptr, &of);
+        if (rc == CWBVH_OK && of) {
+            cw::set_error("traversal stack overflow");
+            rc = CWBVH_ERR_STACK_DEPTH;
+        }
     }
     g_status = rc;
     g_ms = ms;

@@ -286,10 +286,7 @@ constexpr int kLoopQueue = 3;
 constexpr int kOccupancyAuto = 0;
 constexpr int kOccupancyFree = 1;
 constexpr int kOccupancy7 = 7;
-// Automatic choice: launches this large (1 M-triangle spheres, AO rays, closest
-// hit, 6 / 7 waves: 4 M rays 381 / 394 us, 5 M 472 / 478, 6 M 548 / 547, 8 M 721 /
-// 708, 16 M 1285 / 1240; any hit 5 M 415 / 416, 6 M 481 / 477, 8 M 621 / 609).
-constexpr long long kOccupancy7MinRays = 3ll << 21;
+constexpr long long kOccupancy7MinRays = cw::kOccupancy7MinRays;
 // Launches that make their rays from surfels run 5 waves otherwise (same scene,
 // any hit, 5 / 7 waves: 2.9 M rays 349 / 347 us, 4 M 470 / 459, 8.3 M 804 / 766;
 // a 200 k-triangle heightfield 330 / 344, 438 / 444, 854 / 822).
