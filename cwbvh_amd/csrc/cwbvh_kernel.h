@@ -1176,25 +1176,9 @@ int32_t launch_cwbvh_t(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStream_
     auto kernel = cwbvh_trace<ANY, STATS, MULTI, PREFETCH, LOOP, SRC, W7, LDSO, SPREAD>;
     long long grid = cfg.grid_blocks;
     if (!MULTI && !p.persistent) {
-        // Waves of the LDS-only kernels trace their last 16 rays with 4 or 8
-        // lanes each (team_trace), so a launch too small to fill the device
-        // gives each wave only 8 or 16 rays: one latency chain per ray shrinks
-        // from the start.  The limit is 4 waves per SIMD; with more, the teams'
-        // waves queue behind one another (MI355X, AO rays on a 65 k-triangle
-        // heightfield, closest hit, us for 64 / 16 / 8 rays per wave: 1,000
-        // rays 37 / 32 / 21; 32,000 rays 36 / 32 / 28; 48,000 rays 35 / 32 / 43;
-        // 96,000 rays 40 / 69 / 63).  Up to half a wave per SIMD, 4 rays per wave:
-        // the teams of a wave wait for one another's loads (same scene, closest
-        // hit, us for 8 / 4 / 2 rays per wave: 500 rays 20.1 / 17.6 / 17.1, 1,000 20.4
-        // / 18.8 / 18.7, 2,000 20.3 / 20.0 / 19.7; 300 k-triangle soup, 1,000 rays 50.3 /
-        // 49.2 / 52.6, 2,000 50.1 / 48.9 / 48.4, 4,000 50.7 / 51.1 / 55.6)
-        p.rays_per_wave = 64;
-        if (LOOP == kLoopInterleave && !STATS && !W7) {
-            const long long waves = 16ll * cw::device_compute_units();
-            if ((p.n + 3) / 4 <= waves / 8) p.rays_per_wave = 4;
-            else if ((p.n + 7) / 8 <= waves) p.rays_per_wave = 8;
-            else if ((p.n + 15) / 16 <= waves) p.rays_per_wave = 16;
-        }
+        p.rays_per_wave = LOOP == kLoopInterleave && !STATS && !W7
+                              ? cw::team_rays_per_wave(p.n, cw::device_compute_units())
+                              : 64;
         const long long per_block = (long long)p.rays_per_wave * (block / 64);
         grid = ((long long)p.n + per_block - 1) / per_block;
         p.idle_budget = 0x7FFFFFFF;  // nothing to refill from

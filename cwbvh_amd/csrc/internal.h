@@ -8,6 +8,7 @@
 #include <string>
 
 #include "common.h"
+#include "launch_rules.h"
 
 struct cwbvh_scene {
     int32_t kind = CWBVH_KIND_CWBVH;
