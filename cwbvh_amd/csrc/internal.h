@@ -53,23 +53,6 @@ int32_t hip_fail(hipError_t e, const char* what);
 // HBM-bound regime (see cwbvh_trace_config_for_scene).
 constexpr int64_t kCacheResidentBytes = 256ll << 20;
 
-// cwbvh_trace_config.persistent == 2: persistent grid from this many rays up
-// (MI355X, AO rays on a 65 k-triangle heightfield: one ray per thread 0.142
-// against 0.164 ms at 2^19 rays, 0.230 against 0.200 ms at 2^20).
-constexpr int64_t kAutoPersistentRays = 3ll << 18;
-// CWBVH any hit: its shorter rays end with teams of lanes in every wave of a
-// one-ray-per-lane launch, and a persistent grid of short rays queues on its
-// claims.  us one ray per lane / persistent, at 1.05 M rays: AO on 1 M-triangle
-// spheres 110 / 127, on 65 k- and 400 k-triangle heightfields 123 / 126 and 165 /
-// 149, diffuse rays in a 300 k-triangle soup 420 / 429, camera rays 22 / 59; at
-// 1.6 M: 142 / 161, 174 / 167, 229 / 200, 597 / 581, 27 / 68.
-constexpr int64_t kAutoPersistentAnyRays = 5ll << 18;
-// Rays made from surfels: a refill also makes its rays, for few lanes.  us one
-// ray per lane / persistent, any hit, 1 M-triangle spheres and a 200 k-triangle
-// heightfield: 0.8 M rays 113 / 121 and 113 / 127, 1.9 M 234 / 255 and 234 / 237,
-// 2.9 M 339 / 349 and 340 / 330, 4 M 463 / 470 and 467 / 438.
-constexpr int64_t kAutoPersistentSurfelRays = 1ll << 21;
-
 // Launches of the plain interleaved kernels from this many rays up run the 7-wave
 // builds (1 M-triangle spheres, AO rays, closest hit, 6 / 7 waves: 4 M rays 381 /
 // 394 us, 5 M 472 / 478, 6 M 548 / 547, 8 M 721 / 708, 16 M 1285 / 1240; any hit 5

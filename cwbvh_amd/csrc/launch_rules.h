@@ -6,6 +6,37 @@
 
 namespace cw {
 
+// cwbvh_trace_config.persistent == 2: persistent grid from this many rays up
+// (MI355X, AO rays on a 65 k-triangle heightfield: one ray per thread 0.142
+// against 0.164 ms at 2^19 rays, 0.230 against 0.200 ms at 2^20).
+constexpr int64_t kAutoPersistentRays = 3ll << 18;
+// CWBVH any hit: its shorter rays end with teams of lanes in every wave of a
+// one-ray-per-lane launch, and a persistent grid of short rays queues on its
+// claims.  us one ray per lane / persistent, at 1.05 M rays: AO on 1 M-triangle
+// spheres 110 / 127, on 65 k- and 400 k-triangle heightfields 123 / 126 and 165 /
+// 149, diffuse rays in a 300 k-triangle soup 420 / 429, camera rays 22 / 59; at
+// 1.6 M: 142 / 161, 174 / 167, 229 / 200, 597 / 581, 27 / 68.
+constexpr int64_t kAutoPersistentAnyRays = 5ll << 18;
+// Rays made from surfels: a refill also makes its rays, for few lanes.  us one
+// ray per lane / persistent, any hit, 1 M-triangle spheres and a 200 k-triangle
+// heightfield: 0.8 M rays 113 / 121 and 113 / 127, 1.9 M 234 / 255 and 234 / 237,
+// 2.9 M 339 / 349 and 340 / 330, 4 M 463 / 470 and 467 / 438.
+constexpr int64_t kAutoPersistentSurfelRays = 1ll << 21;
+
+// The line of a launch.  Only kernels with teams of lanes gain from the later
+// lines: without them a wave lasts as long as its slowest ray (400 k-triangle
+// heightfield, us one ray per lane / persistent, any hit, 1 M AO rays: grouped 278 /
+// 229, speculative 247 / 208; 2 M surfel rays, closest hit: 454 / 415, 450 / 342).  Nor
+// does any hit in a scene that streams from memory, where a wave's last rays wait on
+// loads that teams do not shorten (diffuse rays, 1.3 M: 5 M-triangle soup 1584 / 1358,
+// 20 M-triangle soup 1957 / 1578; rays made from surfels in the former at 1.06 M 324 /
+// 331, 2 M 585 / 571).
+constexpr int64_t auto_persistent_rays(bool any, bool surfels, bool teams, bool streams) {
+    if (!teams) return kAutoPersistentRays;
+    if (surfels) return kAutoPersistentSurfelRays;
+    return any && !streams ? kAutoPersistentAnyRays : kAutoPersistentRays;
+}
+
 // Rays per wave of a CWBVH launch without work fetching, for kernels whose waves
 // trace their last 16 rays with 4 or 8 lanes each (team_trace): a launch too
 // small to fill the device gives each wave only 8 or 16 rays, so that one latency

@@ -645,6 +645,14 @@ static bool lds_only(const cwbvh_scene* s, const cwbvh_trace_config& c) {
     return s->stack_need > 0 && s->stack_need <= c.lds_depth && c.lds_depth <= kStackCapacity;
 }
 
+// Persistent grid or one ray per lane; configuration value 2 = automatic: below
+// the line the grid's fixed start-up and exit cost outweighs its load balancing.
+static int persistent_grid(const TraceLaunch& L, bool surfels) {
+    if (L.cfg.persistent != 2) return L.cfg.persistent;
+    const bool teams = L.cfg.loop_mode == kLoopInterleave && !(L.flags & CWBVH_TRACE_STATS) && L.cfg.occupancy != kOccupancy7;
+    return L.n >= auto_persistent_rays((L.flags & CWBVH_TRACE_ANY) != 0, surfels, teams, L.scene->bytes > kCacheResidentBytes);
+}
+
 // The spread nodes of a scene serve its LDS-only interleaved launches (no
 // counters, rays from a buffer, the build for 6 or fewer waves).
 static void choose_nodes(CwbvhParams& p, const TraceLaunch& L) {
@@ -677,12 +685,7 @@ int32_t launch_cwbvh(const TraceLaunch& L) {
     p.postpone_pct = L.cfg.postpone_pct;
     p.prim_id = (L.flags & CWBVH_TRACE_PRIM_ID) ? 1 : 0;
     p.slices = L.cfg.work_slices;
-    // 2 = automatic: below kAutoPersistentRays the persistent grid's fixed
-    // start-up and exit cost outweighs its load balancing (MI355X, AO rays on a
-    // 65 k-triangle heightfield: 262 k rays trace 1.9x faster one per thread,
-    // 1 M rays 15% slower)
-    const int64_t pers_from = (L.flags & CWBVH_TRACE_ANY) ? cw::kAutoPersistentAnyRays : cw::kAutoPersistentRays;
-    p.persistent = L.cfg.persistent == 2 ? (L.n >= pers_from ? 1 : 0) : L.cfg.persistent;
+    p.persistent = persistent_grid(L, false);
     p.spec_limit = cw::speculation_limit(s->stack_need);
     p.lds_only = lds_only(s, L.cfg) ? 1 : 0;
     choose_nodes(p, L);
@@ -722,7 +725,7 @@ int32_t launch_cwbvh_surfels(const TraceLaunch& L) {
     p.postpone_pct = L.cfg.postpone_pct;
     p.prim_id = (L.flags & CWBVH_TRACE_PRIM_ID) ? 1 : 0;
     p.slices = L.cfg.work_slices;
-    p.persistent = L.cfg.persistent == 2 ? (L.n >= cw::kAutoPersistentSurfelRays ? 1 : 0) : L.cfg.persistent;
+    p.persistent = persistent_grid(L, true);
     p.spec_limit = cw::speculation_limit(s->stack_need);
     p.lds_only = lds_only(s, L.cfg) ? 1 : 0;
     p.surf_pos = (const float4*)L.surf_pos;

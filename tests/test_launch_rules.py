@@ -32,3 +32,11 @@ def test_rays_per_wave(check):
     sizes = [(1, 4), (2048, 4), (2049, 8), (32768, 8), (32769, 16), (65536, 16), (65537, 64), (10**9, 64)]
     sizes += [(n - k, 64) for k in range(18)]
     check([(f"team_rays_per_wave({k}, 256)", v) for k, v in sizes])
+
+
+def test_persistent_lines(check):
+    """any hit, rays from surfels, teams of lanes, scene that streams from memory."""
+    plain, any_hit, surfels = 3 << 18, 5 << 18, 1 << 21
+    lines = {(1, 0, 1, 0): any_hit, (0, 1, 1, 0): surfels, (1, 1, 1, 0): surfels, (0, 1, 1, 1): surfels, (1, 1, 1, 1): surfels}
+    every = [tuple(i >> k & 1 for k in range(4)) for i in range(16)]
+    check([("auto_persistent_rays(%d, %d, %d, %d)" % k, lines.get(k, plain)) for k in every])
