@@ -152,6 +152,7 @@ struct CwbvhParams {
     unsigned block_q, block_r;      // total_blocks = block_q * slices + block_r
     int spec_limit;                 // single scene: speculation_limit of its tree
     int lds_only;                   // host side: the tree's stack need fits lds_depth (LDS-only kernels)
+    int streams;                    // host side: the scene is larger than the Infinity Cache
     // SRC = kRaysFromSurfels: generate ray r from surfel r / rays_per_texel
     const float4* __restrict__ surf_pos;
     const float4* __restrict__ surf_nrm;
@@ -283,6 +284,11 @@ constexpr int kLoopQueue = 3;
 // waves) would spill 10 registers or more at 7 waves, and the grouped and
 // speculative schedules serve scenes that stream from HBM, where spills and the
 // extra wave cost more.
+// The grouped kernel is built for 6 waves (76 VGPRs, nothing spilled) beside the
+// free build (83: 5 waves): the former serves scenes that the cache holds, the
+// latter those that stream from memory, where a sixth wave evicts more than it
+// hides.  us, free / 6 waves: 1 M-triangle spheres, AO rays, closest hit, 1 M 254 /
+// 242, 8 M 1449 / 1323; 5 M-triangle soup, 0.3 M rays 719 / 751, 16 M 14370 / 14773.
 constexpr int kOccupancyAuto = 0;
 constexpr int kOccupancyFree = 1;
 constexpr int kOccupancy7 = 7;
@@ -293,7 +299,9 @@ constexpr long long kOccupancy7MinRays = cw::kOccupancy7MinRays;
 constexpr long long kOccupancy7MinSurfelRays = 1ll << 22;
 
 #ifndef CWBVH_TRACE_ATTR
-#define CWBVH_TRACE_ATTR __attribute__((amdgpu_waves_per_eu(W7 ? 7 : LOOP == kLoopInterleave && !STATS && !PREFETCH && SRC == 0 && !MULTI ? 6 : 1)))
+#define CWBVH_TRACE_ATTR                        \
+    __attribute__((amdgpu_waves_per_eu(TIGHT ? (LOOP == kLoopGroup ? 6 : 7) : \
+                                       LOOP == kLoopInterleave && !STATS && !PREFETCH && SRC == 0 && !MULTI ? 6 : 1)))
 #endif
 
 // A wave whose pool is dry traces its last kLastRays rays with teams of lanes
@@ -565,11 +573,11 @@ __device__ __forceinline__ unsigned long long team_trace(const CwbvhParams& P, C
     return __ballot(busy && j == 0);
 }
 
-template <bool ANY, bool STATS, bool MULTI, bool PREFETCH, int LOOP, int SRC = kRaysFromBuffer, bool W7 = false,
+template <bool ANY, bool STATS, bool MULTI, bool PREFETCH, int LOOP, int SRC = kRaysFromBuffer, bool TIGHT = false,
           bool LDSO = false, bool SPREAD = false>
 __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhParams P) {
-    static_assert(!W7 || (LOOP == kLoopInterleave && !MULTI && !STATS && !PREFETCH),
-                  "the 7-wave build is made for the plain interleaved kernels only");
+    static_assert(!TIGHT || (LOOP != kLoopSpeculate && !MULTI && !STATS && !PREFETCH),
+                  "the tight builds are made for the plain interleaved and grouped kernels only");
     // LDSO: the launch's trees (a batch: every job's tree) need at most
     // lds_depth stack entries, so the stack lives in LDS only (interleaved
     // schedule: only node groups are pushed, one per level of the tree)
@@ -582,7 +590,7 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
     constexpr bool kTwoGroups = ANY && LOOP == kLoopInterleave && !STATS;
     constexpr bool kRepeatTriangles = !ANY && !PREFETCH && LOOP == kLoopInterleave && !STATS;
     constexpr bool kLookAhead = !ANY && PREFETCH && LOOP == kLoopInterleave && !STATS;
-    constexpr bool kTeams = LOOP == kLoopInterleave && !STATS && !W7;
+    constexpr bool kTeams = LOOP == kLoopInterleave && !STATS && !TIGHT;
     extern __shared__ unsigned long long lds_stack_raw[];
     CWD_LDS unsigned long long* lds_stack = lds_ptr(lds_stack_raw);
     unsigned long long spill[kStackCapacity];
@@ -1168,15 +1176,15 @@ void set_splits(Params& p) {
     p.block_r = (unsigned)p.total_blocks % sl;
 }
 
-template <bool ANY, bool STATS, bool MULTI, bool PREFETCH, int LOOP, int SRC = kRaysFromBuffer, bool W7 = false,
+template <bool ANY, bool STATS, bool MULTI, bool PREFETCH, int LOOP, int SRC = kRaysFromBuffer, bool TIGHT = false,
           bool LDSO = false, bool SPREAD = false>
 int32_t launch_cwbvh_t(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStream_t stream) {
     const int block = cfg.block_size;
     const size_t lds = (size_t)block * (size_t)cfg.lds_depth * sizeof(unsigned long long);
-    auto kernel = cwbvh_trace<ANY, STATS, MULTI, PREFETCH, LOOP, SRC, W7, LDSO, SPREAD>;
+    auto kernel = cwbvh_trace<ANY, STATS, MULTI, PREFETCH, LOOP, SRC, TIGHT, LDSO, SPREAD>;
     long long grid = cfg.grid_blocks;
     if (!MULTI && !p.persistent) {
-        p.rays_per_wave = LOOP == kLoopInterleave && !STATS && !W7
+        p.rays_per_wave = LOOP == kLoopInterleave && !STATS && !TIGHT
                               ? cw::team_rays_per_wave(p.n, cw::device_compute_units())
                               : 64;
         const long long per_block = (long long)p.rays_per_wave * (block / 64);
@@ -1240,7 +1248,11 @@ int32_t dispatch_loop(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStream_t
             }
             return launch_cwbvh_t<ANY, STATS, MULTI, PREFETCH, kLoopInterleave>(p, cfg, st);
         case kLoopSpeculate: return launch_cwbvh_t<ANY, STATS, MULTI, PREFETCH, kLoopSpeculate>(p, cfg, st);
-        default: return launch_cwbvh_t<ANY, STATS, MULTI, PREFETCH, kLoopGroup>(p, cfg, st);
+        default:
+            if constexpr (!STATS && !MULTI && !PREFETCH) {
+                if (!p.streams) return launch_cwbvh_t<ANY, false, false, false, kLoopGroup, kRaysFromBuffer, true>(p, cfg, st);
+            }
+            return launch_cwbvh_t<ANY, STATS, MULTI, PREFETCH, kLoopGroup>(p, cfg, st);
     }
 }
 

@@ -688,6 +688,7 @@ int32_t launch_cwbvh(const TraceLaunch& L) {
     p.persistent = persistent_grid(L, false);
     p.spec_limit = cw::speculation_limit(s->stack_need);
     p.lds_only = lds_only(s, L.cfg) ? 1 : 0;
+    p.streams = s->bytes > kCacheResidentBytes ? 1 : 0;
     choose_nodes(p, L);
     return dispatch_cwbvh<false>(p, L.flags, L.cfg, L.stream);
 }
