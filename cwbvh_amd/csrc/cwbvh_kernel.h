@@ -1191,7 +1191,10 @@ int32_t launch_cwbvh_t(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStream_
         grid = ((long long)p.n + per_block - 1) / per_block;
         p.idle_budget = 0x7FFFFFFF;  // nothing to refill from
     } else if (grid <= 0) {
-        grid = (long long)resident_blocks(kernel, block, lds) * cw::device_compute_units();
+        grid = resident_blocks(kernel, block, lds);
+        const int waves = cw::grid_waves(!MULTI && PREFETCH, p.order != nullptr, p.streams != 0);
+        if (waves > 0) grid = std::min(grid, (long long)waves * 4 * 64 / block);
+        grid *= cw::device_compute_units();
     }
     p.total_waves = (int)(grid * (block / 64));
     if (MULTI && cfg.grid_blocks <= 0) {

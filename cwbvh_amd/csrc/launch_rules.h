@@ -57,4 +57,14 @@ constexpr int32_t team_rays_per_wave(int64_t n, int32_t compute_units) {
     return 64;
 }
 
+// Waves per SIMD of an automatic persistent grid, 0 = all that fit.  A prefetch
+// launch on rays in the caller's order in a scene that streams from memory runs 4: the
+// rays in flight share few nodes, and those of a fifth wave evict more from the
+// caches than it hides.  (Rays sorted by the launch share many, and from 16 M up 5
+// waves are faster.)  5 / 4 / 3 waves, ms: diffuse rays, 20 M-triangle soup, closest hit,
+// 16 M 16.41 / 15.72 / 15.67, 4 M 4.39 / 4.20 / 4.20, 1 M 1.44 / 1.36 / 1.38; 5 M triangles
+// 13.84 / 13.69 / 13.74, 3.69 / 3.63 / 3.66, 1.18 / 1.14 / 1.17; AO rays in the former 9.90 /
+// 9.69 / 10.51, 2.60 / 2.54 / 2.75, 0.79 / 0.78 / 0.83; any hit alike.
+constexpr int32_t grid_waves(bool prefetch, bool ordered, bool streams) { return prefetch && !ordered && streams ? 4 : 0; }
+
 }  // namespace cw

@@ -40,3 +40,9 @@ def test_persistent_lines(check):
     lines = {(1, 0, 1, 0): any_hit, (0, 1, 1, 0): surfels, (1, 1, 1, 0): surfels, (0, 1, 1, 1): surfels, (1, 1, 1, 1): surfels}
     every = [tuple(i >> k & 1 for k in range(4)) for i in range(16)]
     check([("auto_persistent_rays(%d, %d, %d, %d)" % k, lines.get(k, plain)) for k in every])
+
+
+def test_waves_of_a_persistent_grid(check):
+    """prefetch, ordered, scene that streams from memory."""
+    every = [tuple(i >> k & 1 for k in range(3)) for i in range(8)]
+    check([("grid_waves(%d, %d, %d)" % k, 4 if k == (1, 0, 1) else 0) for k in every])
