@@ -60,8 +60,6 @@ struct Bvh2Params {
     int lds_depth;
     int woop_last;   // last valid float4 index of tris (loads past a leaf terminator clamp here)
     int prim_id;
-    int share;       // bvh2_trace: rays per wave
-    int in_l2;       // host side: the scene fits one XCD's L2
     // persistent launches (bvh2_trace_persistent) only
     int slices;
     int chunk;
@@ -70,6 +68,11 @@ struct Bvh2Params {
     int total_blocks;
     unsigned item_q, item_r;   // n = item_q * slices + item_r
     unsigned block_q, block_r; // total_blocks = block_q * slices + block_r
+    // not read by the persistent kernel, so behind its fields: before them they moved
+    // those into one more 64-byte line of arguments, which its short launches, most of
+    // whose time is their waves' start, paid with 20 us (3,000 rays 223 us, 206 so)
+    int share;       // bvh2_trace: rays per wave
+    int in_l2;       // host side: the scene fits one XCD's L2
 };
 
 // Slab test of one BVH2 child box (reference src/TraversalKernelBVH2.cu:14-24).
