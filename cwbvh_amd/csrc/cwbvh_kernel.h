@@ -152,7 +152,6 @@ struct CwbvhParams {
     unsigned block_q, block_r;      // total_blocks = block_q * slices + block_r
     int spec_limit;                 // single scene: speculation_limit of its tree
     int lds_only;                   // host side: the tree's stack need fits lds_depth (LDS-only kernels)
-    int streams;                    // host side: the scene is larger than the Infinity Cache
     // SRC = kRaysFromSurfels: generate ray r from surfel r / rays_per_texel
     const float4* __restrict__ surf_pos;
     const float4* __restrict__ surf_nrm;
@@ -161,6 +160,7 @@ struct CwbvhParams {
     float gen_tmin, gen_tmax;
     unsigned long long seed;
     unsigned* texel_hits;           // non-null: count hits per surfel instead of writing hits
+    int streams;                    // host side: the scene is larger than the Infinity Cache
 };
 
 constexpr int kRaysFromBuffer = 0;
