@@ -53,7 +53,7 @@ void bind(cwbvh_scene*& slot, int32_t kind, int32_t stride, const cwbvh_float4* 
 constexpr int32_t kBoundLdsDepth = 12;
 
 bool bound_config(const cwbvh_scene* scene, int count, cwbvh_trace_config* cfg) {
-    if (scene->kind != CWBVH_KIND_CWBVH || count >= cw::kOccupancy7MinRays) return false;
+    if (scene->kind != CWBVH_KIND_CWBVH || count >= cw::seven_wave_rays(false, false)) return false;
     if (cwbvh_trace_config_for_scene(scene, cfg) != CWBVH_OK || cfg->prefetch || cfg->loop_mode != 1) return false;
     cfg->lds_depth = kBoundLdsDepth;
     return true;

@@ -302,7 +302,6 @@ constexpr int kLoopQueue = 3;
 constexpr int kOccupancyAuto = 0;
 constexpr int kOccupancyFree = 1;
 constexpr int kOccupancy7 = 7;
-constexpr long long kOccupancy7MinRays = cw::kOccupancy7MinRays;
 // Launches that make their rays from surfels run 5 waves otherwise (same scene,
 // any hit, 5 / 7 waves: 2.9 M rays 349 / 347 us, 4 M 470 / 459, 8.3 M 804 / 766;
 // a 200 k-triangle heightfield 330 / 344, 438 / 444, 854 / 822).
@@ -1250,7 +1249,7 @@ int32_t dispatch_loop(CwbvhParams& p, const cwbvh_trace_config& cfg, hipStream_t
         case kLoopInterleave:
             if constexpr (!STATS && !MULTI) {
                 const bool w7 = !PREFETCH && (cfg.occupancy == kOccupancy7 ||
-                                              (cfg.occupancy == kOccupancyAuto && (long long)p.n >= kOccupancy7MinRays));
+                                              (cfg.occupancy == kOccupancyAuto && p.n >= cw::seven_wave_rays(ANY, p.lds_only != 0)));
                 if (p.lds_only) {
                     if (w7) return launch_cwbvh_t<ANY, false, false, false, kLoopInterleave, kRaysFromBuffer, true, true>(p, cfg, st);
                     if (p.spread) return launch_cwbvh_t<ANY, false, false, PREFETCH, kLoopInterleave, kRaysFromBuffer, false, true, true>(p, cfg, st);

@@ -53,12 +53,6 @@ int32_t hip_fail(hipError_t e, const char* what);
 // HBM-bound regime (see cwbvh_trace_config_for_scene).
 constexpr int64_t kCacheResidentBytes = 256ll << 20;
 
-// Launches of the plain interleaved kernels from this many rays up run the 7-wave
-// builds (1 M-triangle spheres, AO rays, closest hit, 6 / 7 waves: 4 M rays 381 /
-// 394 us, 5 M 472 / 478, 6 M 548 / 547, 8 M 721 / 708, 16 M 1285 / 1240; any hit 5
-// M 415 / 416, 6 M 481 / 477, 8 M 621 / 609).
-constexpr int64_t kOccupancy7MinRays = 3ll << 21;
-
 constexpr int kWorkSlices = 8;
 constexpr int kWorkStride = 64;                       // uint32 per counter line
 constexpr int kWorkExited = kWorkSlices * kWorkStride;

@@ -57,6 +57,15 @@ constexpr int32_t team_rays_per_wave(int64_t n, int32_t compute_units) {
     return 64;
 }
 
+// Rays from which launches of the plain interleaved kernels run the 7-wave builds
+// (1 M-triangle spheres, AO rays, closest hit, 6 / 7 waves: 4 M rays 381 / 394 us, 5 M
+// 472 / 478, 6 M 548 / 547, 8 M 721 / 708, 16 M 1285 / 1240; any hit 5 M 415 / 416, 6 M
+// 481 / 477, 8 M 621 / 609).  Any hit with a two-level stack, whose 6-wave build is the
+// slower of the two kinds, earlier (4.3 M rays 487 / 467, 5.5 M 605 / 576; heightfields of
+// 65 k and 2 M triangles 399 / 400 and 589 / 602, 498 / 487 and 732 / 746; closest hit 567 /
+// 567, 698 / 703, 455 / 477, 660 / 713).
+constexpr int64_t seven_wave_rays(bool any, bool lds_only) { return any && !lds_only ? 1ll << 22 : 3ll << 21; }
+
 // Waves per SIMD of an automatic persistent grid, 0 = all that fit.  A prefetch
 // launch on rays in the caller's order in a scene that streams from memory runs 4: the
 // rays in flight share few nodes, and those of a fifth wave evict more from the

@@ -661,7 +661,7 @@ static int persistent_grid(const TraceLaunch& L, bool surfels) {
 static void choose_nodes(CwbvhParams& p, const TraceLaunch& L) {
     const cwbvh_trace_config& c = L.cfg;
     const bool w7 = !c.prefetch && (c.occupancy == kOccupancy7 ||
-                                    (c.occupancy == kOccupancyAuto && (long long)L.n >= kOccupancy7MinRays));
+                                    (c.occupancy == kOccupancyAuto && L.n >= seven_wave_rays((L.flags & CWBVH_TRACE_ANY) != 0, true)));
     p.spread = p.lds_only && L.scene->spread_nodes && c.loop_mode == kLoopInterleave && !w7 && !(L.flags & CWBVH_TRACE_STATS);
     if (p.spread) p.nodes = (const float4*)L.scene->spread_nodes;
 }

@@ -117,3 +117,14 @@ def test_bvh2(cw, rays, any_hit):
     rays.grow(BVH2_BLOCKS + 1)
     for n in around(BVH2_L2_BLOCKS, BVH2_BLOCKS):
         rays.check("bvh2", any_hit, n, lambda n, fl: sc.trace(rays.d_rays.ptr, rays.d_hits.ptr, n, fl), "default")
+
+
+@pytest.mark.parametrize("any_hit", [False, True])
+def test_unknown_need(cw, rays, any_hit):
+    """Arrays of unknown stack need: any hit runs 7 waves from 2^22 rays up, closest hit from 3 x 2^21."""
+    lay = rays.cwbvh
+    bufs = [cw.DeviceBuffer.from_numpy(a) for a in (lay.nodes, lay.woop, lay.prim_idx)]
+    sc = cw.Scene.wrap(lay.kind, lay.node_stride, bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, 0, keep=bufs)
+    for n in around(1 << 22, SEVEN_WAVES):
+        rays.check("cwbvh", any_hit, n, lambda n, fl: sc.trace(rays.d_rays.ptr, rays.d_hits.ptr, n, fl), "unknown need")
+    assert not cw.stack_overflowed()

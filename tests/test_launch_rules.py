@@ -46,3 +46,7 @@ def test_waves_of_a_persistent_grid(check):
     """prefetch, ordered, scene that streams from memory."""
     every = [tuple(i >> k & 1 for k in range(3)) for i in range(8)]
     check([("grid_waves(%d, %d, %d)" % k, 4 if k == (1, 0, 1) else 0) for k in every])
+
+
+def test_seven_wave_lines(check):
+    check([("seven_wave_rays(%d, %d)" % k, 1 << 22 if k == (1, 0) else 3 << 21) for k in ((0, 0), (0, 1), (1, 0), (1, 1))])
