@@ -30,13 +30,10 @@ constexpr int kWorkProfile = cw::kWorkProfile;
 constexpr int kWorkDrained = cw::kWorkDrained;
 constexpr int kWorkGroupExit = cw::kWorkGroupExit;
 
-// Work distribution of the persistent single-scene grids (cwbvh_trace,
-// bvh2_trace_persistent).  The rays are split into `slices` contiguous ranges
-// with one claim counter each.  Blocks are dispatched round-robin over the
+// Work distribution of the persistent grids (cwbvh_trace, bvh2_trace_persistent).
+// The items (rays; in a batch, chunk indices) are split into `slices` contiguous
+// ranges with one claim counter each.  Blocks are dispatched round-robin over the
 // XCDs, so block b takes slice b % slices (its home) first, then the others.
-// (Batches claim chunk indices with a plain atomic per claim and count exits
-// on one word: with the three changes below their kernel ran 6% slower on
-// 32 scenes of 1 M rays each.)
 //  * First claim without an atomic: wave i of the W_s waves whose home is
 //    slice s owns [i * amount, (i + 1) * amount) of it outright, and the
 //    counter hands out the slice from W_s * amount on.  Otherwise every wave
@@ -285,15 +282,13 @@ constexpr int kLoopQueue = 3;
 // Register budget (cwbvh_trace_config.occupancy).  The plain interleaved
 // kernels (one scene, no counters, no prefetch) that read rays from a buffer are
 // held to 6 waves: team_trace's code would lift them from 76 to 83 VGPRs, i.e. to
-// 5; held, they take 75-78 and spill nothing.  Those that make rays from surfels
-// take 84-89 (5 waves).  Both are also built for 7 waves (72 VGPRs; up to 1 and 6
+// 5; held, they take 77-78 and spill nothing.  Those that make rays from surfels
+// take 84-89 (5 waves).  Both are also built for 7 waves (72 VGPRs; up to 1 and 7
 // registers of cold state spilled), which traces launches of tens of millions of
 // AO rays 3-5% faster and launches of a million rays 6-7% slower (more waves,
-// each slower, lengthen the tail of a short launch).  The other instances stay
-// unconstrained: the batch kernels (84-89) and the prefetch kernels (93-96, 5
-// waves) would spill 10 registers or more at 7 waves, and the grouped and
-// speculative schedules serve scenes that stream from HBM, where spills and the
-// extra wave cost more.
+// each slower, lengthen the tail of a short launch).  The batch kernels (85-94) and
+// the prefetch kernels (90-96), 5 waves both, stay unconstrained: at 7 waves they
+// would spill 10 registers or more.
 // The grouped kernel is built for 6 waves (76 VGPRs, nothing spilled) beside the
 // free build (83: 5 waves): the former serves scenes that the cache holds, the
 // latter those that stream from memory, where a sixth wave evicts more than it
@@ -592,8 +587,8 @@ __global__ __launch_bounds__(kMaxBlock) CWBVH_TRACE_ATTR void cwbvh_trace(CwbvhP
     // schedule: only node groups are pushed, one per level of the tree)
     static_assert(!LDSO || (LOOP == kLoopInterleave && !STATS), "LDS-only stacks serve the interleaved schedule");
     static_assert(!SPREAD || (LDSO && !MULTI), "spread nodes serve the LDS-only single-scene kernels");
-    // The last rays of a wave go to teams of lanes (team_trace) where the stack
-    // is in LDS.  The 7-wave builds serve launches of 3 x 2^21 rays and more, whose
+    // The last rays of a wave go to teams of lanes (team_trace), with a two-level
+    // stack once none of them has entries in scratch.  The 7-wave builds serve launches of 3 x 2^21 rays and more, whose
     // tail is 3% of their time; with team_trace their node loop spills scalars
     // and they run 2.3% slower (33 M AO rays: 2.19 against 2.14 ms).
     constexpr bool kTwoGroups = ANY && LOOP == kLoopInterleave && !STATS;

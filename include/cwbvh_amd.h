@@ -344,7 +344,8 @@ typedef struct cwbvh_trace_config {
     int32_t block_size;      /* 64, 128 or 256 threads (BVH2 with one ray per lane: 64, except from
                                 3 x 2^23 rays up, scenes up to 4 MB from 2^20) */
     int32_t lds_depth;       /* stack entries per lane kept in LDS (1..stack capacity) */
-    int32_t grid_blocks;     /* persistent grid (0 = fill the device) */
+    int32_t grid_blocks;     /* persistent grid (0 = fill the device; CWBVH prefetch launches on rays in the
+                                given order in scenes larger than 256 MB: 4 waves per SIMD) */
     int32_t fetch_chunk;     /* rays claimed per wave-level atomic (persistent grids; 0 = automatic: 64..512
                                 by the launch's rays per wave, 64 with a ray order, 32 with prefetch;
                                 batches 8..256) */
@@ -358,8 +359,9 @@ typedef struct cwbvh_trace_config {
     int32_t work_slices;     /* 1..8 contiguous ray ranges, one drained first per XCD (persistent grids) */
     int32_t persistent;      /* 1 = persistent grid with work fetching, 0 = one ray per lane (launches too
                                 small to fill the device: fewer rays per wave, CWBVH 4, 8, 16 or 64, BVH2 1 to
-                                16 or 64), 2 = persistent from 786,432 (3 x 2^18) rays up, CWBVH any hit
-                                from 1,310,720 (5 x 2^18), rays made from surfels from 2,097,152 (2^21).
+                                16 or 64), 2 = persistent from 786,432 (3 x 2^18) rays up; with loop_mode 1,
+                                no STATS and occupancy not 7, rays made from surfels from 2,097,152 (2^21),
+                                any hit in scenes of up to 256 MB from 1,310,720 (5 x 2^18).
                                 CWBVH default 2.  BVH2 default 0 (the reference's kernel); its persistent grid hands rays to idle lanes
                                 between while-while rounds and uses grid_blocks, fetch_chunk,
                                 refill_idle (>= 0), refill_budget (>= 1) and work_slices.  BVH2
@@ -372,7 +374,8 @@ typedef struct cwbvh_trace_config {
                                 queue) was taken out and is refused with CWBVH_ERR_INVALID_ARGUMENT */
     int32_t occupancy;       /* register budget of the single-scene loop_mode 1 kernels (no prefetch,
                                 no stats; rays from a buffer or from surfels): 0 = automatic
-                                (7 waves per SIMD for launches of 3 x 2^21 rays or more, from surfels 2^22), 1 = unconstrained,
+                                (7 waves per SIMD for launches of 3 x 2^21 rays or more; from surfels, and any hit
+                                with a stack partly in scratch, 2^22), 1 = unconstrained,
                                 7 = 7 waves per SIMD (72 VGPRs) */
     int32_t ray_order;       /* 0 = trace rays in the given order; 1 = a launch of 2^20 rays or more
                                 first sorts them by direction octant and origin Morton code (as
